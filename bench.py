@@ -33,17 +33,17 @@ NVAR = 10
 #   transverse_1: per d-face: qm, qp (18), two transverse fluxes +
 #     Godunov of its cell (2 x 10), sound speed / floor (2); writes two
 #     compact fluxes + Godunov (2 x 10) = 60 doubles.
-#   trace_ppm: per cell: compact primitives (9 + sound speed) and flat (1);
-#     writes the two face states (2 x 9) = 29 doubles.
-#   riemann_normal: per face: qm, qp (18), sound speed / floor of both
-#     cells (2); writes the compact flux + Godunov (10) = 30 doubles.
+#   trace_riemann (one launch, all three directions): per face: the cell's
+#     compact primitives (9 + sound speed / floor) and flat (1); writes the
+#     two face states (2 x 9) and the compact flux + Godunov (10)
+#     = 40 doubles.
 #   transverse_ctu (the CTU face kernels, transdo pairs + transdd + final
 #     solve of one direction): per d-face: qm, qp of all three directions
 #     (54), the first fluxes + Godunov of the two transverse directions
 #     (20), sound speed / floor (2), conserved state (10), one divu node;
 #     writes the final flux and Godunov (12) = 99 doubles.
-ALGO_DOUBLES = {"transverse_2": 63, "transverse_1": 60, "trace_ppm": 29,
-                "riemann_normal": 30, "transverse_ctu": 99}
+ALGO_DOUBLES = {"transverse_2": 63, "transverse_1": 60,
+                "trace_riemann": 40, "transverse_ctu": 99}
 # mol_faces (one launch per direction d, method of lines, flux adjustment
 # fused): per d-face, the 9 primitives and 3 aux values (c, csmall, gamma)
 # of one cell, its 10 conserved values (artificial viscosity) and one divu
@@ -70,13 +70,13 @@ FP64_EXECUTED_PER_CELL_UPDATE = 10069
 # (`python oracle/count_ops.py --n 256`, profiles/fp64_opcount_256cube_ppm.md).
 # Keys are the profiler regions of the fused engine; a face stage's count
 # covers its three launches (one per direction).
-ALGO_FLOP = {"fill_clean_prim": 169.0, "flatten": 59.3, "trace_ppm": 3501.9,
-             "riemann_normal": 300.6, "transverse_1": 1285.1, "divu": 30.4,
+ALGO_FLOP = {"fill_clean_prim": 169.0, "flatten": 59.3,
+             "trace_riemann": 3501.9 + 300.6, "transverse_1": 1285.1, "divu": 30.4,
              "transverse_2": 989.9, "consup_clean_estdt": 111.0 + 129.0}
 ALGO_FLOP_PER_CELL_UPDATE = sum(ALGO_FLOP.values())
 # the CTU face kernels do the work of both transverse stages
 ALGO_FLOP["transverse_ctu"] = ALGO_FLOP["transverse_1"] + ALGO_FLOP["transverse_2"]
-LAUNCHES_PER_STEP = {"trace_ppm": 3, "riemann_normal": 3, "transverse_1": 3,
+LAUNCHES_PER_STEP = {"transverse_1": 3,
                      "transverse_2": 3, "transverse_ctu": 3}
 
 
@@ -86,10 +86,8 @@ def unit_count(name: str, n: int) -> int:
         return (n + 1) * n * n
     if name.startswith("transverse_1"):
         return (n + 3) * (n + 2) * (n + 2)
-    if name.startswith("trace_ppm"):
-        return (n + 4) ** 3
-    if name.startswith("riemann_normal"):
-        return (n + 3) * (n + 4) * (n + 4)
+    if name.startswith("trace_riemann"):
+        return 3 * (n + 3) * (n + 4) * (n + 4)
     return n ** 3
 
 

@@ -53,8 +53,8 @@ CANDIDATES = tuple((bs, LINEAR, k) for bs in BLOCKS for k in XCD_CHUNKS) + tuple
 # profiler region name -> stage-range indices (CAMR_NSTAGE order)
 STAGES = {
     "fill_clean_prim": (0,), "prim": (0,),
-    "flatten": (1,), "trace_ppm": (1,), "trace_plm": (1,),
-    "riemann_normal": (2, 3, 4),
+    "flatten": (1,),
+    "trace_riemann": (2, 3, 4),  # only the XCD chunk: the stage has its own blocks
     "transverse_1": (5, 6, 7),
     "divu": (8,),
     "transverse_2": (9, 10, 11),

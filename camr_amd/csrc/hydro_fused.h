@@ -165,11 +165,11 @@ __host__ __device__ inline int64_t batch_blocks(const Box &sb, int block, int lx
 // With B.xk = K the launch's blocks are permuted within groups of 8K: the
 // workgroups of one XCD take K consecutive logical blocks, while all XCDs
 // stay within the same window of 8K blocks (the same few planes).
-__device__ __forceinline__ int batch_box(const Batch &B, int &lblock) {
-    int w = (int)blockIdx.x;
+// w is the block of the nw blocks that the launch has for this batch.
+__device__ __forceinline__ int batch_box(const Batch &B, int w, int nw, int &lblock) {
     if (B.xk > 0) {
         const int g = 8 * B.xk;
-        if (w < ((int)gridDim.x / g) * g) {
+        if (w < (nw / g) * g) {
             const int r = w % g;
             w = (w - r) + (r & 7) * B.xk + (r >> 3);
         }
@@ -184,6 +184,27 @@ __device__ __forceinline__ int batch_box(const Batch &B, int &lblock) {
     lblock = bid - B.blk[lo];
     return lo;
 }
+__device__ __forceinline__ int batch_box(const Batch &B, int &lblock) {
+    return batch_box(B, (int)blockIdx.x, (int)gridDim.x, lblock);
+}
+
+// The three directions of a face stage in one launch: blocks [end[d-1],
+// end[d]) are direction d's, with its own prefix table and block shape.
+struct Batch3 {
+    Batch d[3];
+    int end[3];
+};
+// Runs BODY<D>(batch, block, blocks, args...) for this block's direction.
+#define BATCH3_DISPATCH(T, BODY, ...)                                          \
+    do {                                                                       \
+        const int w_ = (int)blockIdx.x;                                        \
+        if (w_ < (T).end[0])                                                   \
+            BODY<0>((T).d[0], w_, (T).end[0], __VA_ARGS__);                    \
+        else if (w_ < (T).end[1])                                              \
+            BODY<1>((T).d[1], w_ - (T).end[0], (T).end[1] - (T).end[0], __VA_ARGS__); \
+        else                                                                   \
+            BODY<2>((T).d[2], w_ - (T).end[1], (T).end[2] - (T).end[1], __VA_ARGS__); \
+    } while (0)
 
 // The point (i,j,k) of stage range sb that this thread covers as the
 // lblk-th block of its box; false past the range's end.  Tiled blocks take
@@ -261,6 +282,20 @@ __device__ __forceinline__ CtuTile ctu_tile(const Box &sb, int lblk, int planes,
     return t;
 }
 
+// Blocks of the trace + first-flux stage of direction d over box bx (see
+// k_face1).  The cells of grow(bx, 2) give the faces above their first one
+// along d.  x: blocks of 256 consecutive cells in x-fastest order, each
+// overlapping the one before by a cell; y, z: kF1Rows cells along d by
+// kF1Cols points across, consecutive tiles along d sharing a cell.
+constexpr int kF1Rows = 16, kF1Cols = kBlock / kF1Rows;
+__host__ __device__ inline int64_t face1_blocks(const Box &bx, int d) {
+    const Box g = grow(bx, 2);
+    if (d == 0) return (g.npts() - 1 + kBlock - 2) / (kBlock - 1);
+    const int64_t across = g.npts() / g.len(d);
+    return ((across + kF1Cols - 1) / kF1Cols) *
+           ((g.len(d) - 1 + kF1Rows - 2) / (kF1Rows - 1));
+}
+
 #define BATCH_COLUMN(KIND)                                                     \
     if (B.halt && *B.halt) return;                                             \
     int lblk_;                                                                 \
@@ -270,11 +305,13 @@ __device__ __forceinline__ CtuTile ctu_tile(const Box &sb, int lblk, int planes,
     if (!batch_column(B, stage_box((KIND), E.bx), lblk_, i, j, k0, k1)) return;
 
 // First statements of every kernel: the block's box E (and its layout L)
-// and the point (i,j,k) of the stage range this thread covers.
-#define BATCH_POINT(KIND)                                                      \
+// and the point (i,j,k) of the stage range this thread covers; _AT: as
+// block W of the NW blocks of batch B.
+#define BATCH_POINT(KIND) BATCH_POINT_AT(KIND, (int)blockIdx.x, (int)gridDim.x)
+#define BATCH_POINT_AT(KIND, W, NW)                                            \
     if (B.halt && *B.halt) return;                                             \
     int lblk_;                                                                 \
-    const BoxEnt &E = B.tab[batch_box(B, lblk_)];                              \
+    const BoxEnt &E = B.tab[batch_box(B, (W), (NW), lblk_)];                   \
     const Canon L = E.L;                                                       \
     int i, j, k;                                                               \
     if (!batch_point(B, stage_box((KIND), E.bx), lblk_, i, j, k)) return;
@@ -438,6 +475,14 @@ class FusedEngine {
     template <typename K, typename... A>
     void launch(const char *name, Prof *prof, K kern, int kind, int b, int parity,
                 hipStream_t st, A... args);
+    // the three directions of stage kind (+0, +1, +2) in one launch
+    template <typename K, typename... A>
+    void launch3(const char *name, Prof *prof, K kern, const LaunchCfg c[3], hipStream_t st,
+                 A... args);
+    // block-prefix row rk (see kBlkRows), table entry range of box b
+    LaunchCfg cfg_row(int rk, int b, int parity) const;
+    // grid of the trace + first-flux kernel of direction d
+    LaunchCfg cfg_face1(int d, int b, int parity) const;
     // grid of the CTU face kernel of direction d
     LaunchCfg cfg_ctu(int d, int b, int parity) const;
     template <typename K, typename... A>
@@ -449,7 +494,8 @@ class FusedEngine {
     std::vector<Arr> bufA_, bufB_;
     std::vector<size_t> off_;      // scratch offset of each box (doubles)
     std::vector<int> order_;       // box order of the tables
-    // (2 x ST_COUNT + 3) x (nbox + 1): as tuned, without z-march, CTU tiles
+    // (2 x ST_COUNT + 6) x (nbox + 1): as tuned, without z-march, CTU tiles,
+    // trace + first-flux tiles
     std::vector<int> blk_host_;
     std::vector<int> pos_;         // table position of box b
     Tuning tune_{};

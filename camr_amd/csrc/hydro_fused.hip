@@ -5,8 +5,8 @@
 // or final interface state ever goes to HBM:
 //   k_prim_c    U -> compact primitives (rho u v w p rhoe Y0..2 c csml)
 //   k_flat_c    shock flattening coefficient
-//   k_ppm_c / k_plm_c   normal predictor states, face-indexed
-//   k_riemann1  first fluxes (with the reference's boundary-face mutation)
+//   k_face1     normal predictor states, face-indexed, and the first fluxes
+//               (with the reference's boundary-face mutation)
 //   k_trans1<D> per D-face: the two transdo states of each side are formed
 //               in registers and solved at once (both pairs D|t)
 //   k_trans2<D> per D-face: transdd states, final Riemann solve, artificial
@@ -165,29 +165,28 @@ k_flat_c(Batch B, int use_flattening, int qgrow, const DevFab *sb_tab, HydroCons
     flat.st(v0, 0, f);
 }
 
-// ------------------------------------------------------------ PPM trace
-// trace_ppm (PPM.cpp:11-411) for direction D; qp(i) is the plus state of
-// face i, qm(i+1) the minus state of face i+1.
+// ------------------------------------------------------------ traces
+// trace_ppm (PPM.cpp:11-411) of the cell at offset v0 for direction D: op
+// is the plus state of the cell's low face, om the minus state of its high
+// face.
 template <int D>
-__global__ void __launch_bounds__(kBlock)
-k_ppm_c(Batch B, HydroConst hc, const double *dtp) {
-    BATCH_POINT(ST_G2)
-    const double dtdx = *dtp / hc.dx[D];
-    const CView q = cview(L, slot_ptr<S_Q>(E), NQC), flat = cview(L, slot_ptr<S_FLAT>(E), 1);
-    const CView qm = cview(L, slot_ptr<S_QM0 + D>(E), NS), qp = cview(L, slot_ptr<S_QP0 + D>(E), NS);
+__device__ __forceinline__ void ppm_cell(const CView &q, unsigned v0, unsigned sd, double fl,
+                                         double cc, double dtdx, const HydroConst &hc,
+                                         double *op, double *om) {
     constexpr int SN = SU + D;
     constexpr int T1 = (D == 0) ? SV : SU;
     constexpr int T2 = (D == 2) ? SV : SW;
-    const unsigned v0 = L.off(i, j, k), sd = shift<D>(L);
-    const double cc = q.ld(v0, SC);
-    const double un = q.ld(v0, SN);
-    const double fl = flat.ld(v0, 0);
     double Ip[NS][3], Im[NS][3];
+    // every load of the stencil before the arithmetic (see F1_BOUNDS)
+    double all[NS][5];
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int o = -2; o <= 2; ++o) all[s][o + 2] = q.ld(v0 + (unsigned)o * sd, s);
+    const double un = all[SN][2];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        double st[5];
-#pragma unroll
-        for (int o = -2; o <= 2; ++o) st[o + 2] = q.ld(v0 + (unsigned)o * sd, s);
+        const double *st = all[s];
         double sm, sp;
         ppm_edges(st, fl, sm, sp);
         const double s6 = ppm_s6(sm, sp, st[2]);
@@ -201,42 +200,29 @@ k_ppm_c(Batch B, HydroConst hc, const double *dtp) {
         W.rho[w] = Im[SR][w]; W.un[w] = Im[SN][w]; W.p[w] = Im[SP][w];
         W.rhoe[w] = Im[SE][w]; W.gam[w] = kGamma;
     }
-    {
-        double ro, uo, po, eo;
-        ppm_project(+1, W, un, cc, hc.small_dens, hc.small_pres, ro, uo, po, eo);
-        qp.st(v0, SR, ro); qp.st(v0, SN, uo); qp.st(v0, SP, po); qp.st(v0, SE, eo);
-        qp.st(v0, T1, Im[T1][1]); qp.st(v0, T2, Im[T2][1]);
+    ppm_project(+1, W, un, cc, hc.small_dens, hc.small_pres, op[SR], op[SN], op[SP], op[SE]);
+    op[T1] = Im[T1][1];
+    op[T2] = Im[T2][1];
 #pragma unroll
-        for (int s = 0; s < NSPEC; ++s) qp.st(v0, SY + s, Im[SY + s][1]);
-    }
+    for (int s = 0; s < NSPEC; ++s) op[SY + s] = Im[SY + s][1];
 #pragma unroll
     for (int w = 0; w < 3; ++w) {
         W.rho[w] = Ip[SR][w]; W.un[w] = Ip[SN][w]; W.p[w] = Ip[SP][w];
         W.rhoe[w] = Ip[SE][w];
     }
-    {
-        double ro, uo, po, eo;
-        ppm_project(-1, W, un, cc, hc.small_dens, hc.small_pres, ro, uo, po, eo);
-        const unsigned v1 = v0 + sd;
-        qm.st(v1, SR, ro); qm.st(v1, SN, uo); qm.st(v1, SP, po); qm.st(v1, SE, eo);
-        qm.st(v1, T1, Ip[T1][1]); qm.st(v1, T2, Ip[T2][1]);
+    ppm_project(-1, W, un, cc, hc.small_dens, hc.small_pres, om[SR], om[SN], om[SP], om[SE]);
+    om[T1] = Ip[T1][1];
+    om[T2] = Ip[T2][1];
 #pragma unroll
-        for (int s = 0; s < NSPEC; ++s) qm.st(v1, SY + s, Ip[SY + s][1]);
-    }
+    for (int s = 0; s < NSPEC; ++s) om[SY + s] = Ip[SY + s][1];
 }
 
-// ------------------------------------------------------------ PLM trace
-// hydro_plm_d (PLM.H:170-323) for direction D.
+// hydro_plm_d (PLM.H:170-323) of the cell, as ppm_cell.
 template <int D>
-__global__ void __launch_bounds__(kBlock)
-k_plm_c(Batch B, int has_src, HydroConst hc, const double *dtp) {
-    BATCH_POINT(ST_G2)
-    const double dtdx = *dtp / hc.dx[D];
-    const CView q = cview(L, slot_ptr<S_Q>(E), NQC), flat = cview(L, slot_ptr<S_FLAT>(E), 1);
-    const CView qm = cview(L, slot_ptr<S_QM0 + D>(E), NS), qp = cview(L, slot_ptr<S_QP0 + D>(E), NS);
-    const CView sq = cview(L, slot_ptr<S_SRCQ>(E), NS);
-    const unsigned v0 = L.off(i, j, k), sd = shift<D>(L);
-    const double fl = flat.ld(v0, 0);
+__device__ __forceinline__ void plm_cell(const CView &q, const CView &sq, int has_src,
+                                         unsigned v0, unsigned sd, double fl, double cc,
+                                         double dtdx, const HydroConst &hc, double *op,
+                                         double *om) {
     double c[NS], sl[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
@@ -256,13 +242,7 @@ k_plm_c(Batch B, int has_src, HydroConst hc, const double *dtp) {
             sl[s] = mc_slope(st, fl, hc.plm_iorder);
         }
     }
-    double op[NS], om[NS];
-    plm_trace(D, c, sl, q.ld(v0, SC), dtdx, hc.small_dens, hc.small_pres, op, om);
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        qp.st(v0, s, op[s]);
-        qm.st(v0 + sd, s, om[s]);
-    }
+    plm_trace(D, c, sl, cc, dtdx, hc.small_dens, hc.small_pres, op, om);
 }
 
 // sound speeds of the cells left (offset vl) and right (vr) of a face
@@ -303,35 +283,120 @@ __device__ __forceinline__ void store_tflux(const CView &F, unsigned v, const do
     F.st(v, TGP, g[GP]);
 }
 
-// ------------------------------------------------------------ first fluxes
-// hydro_cmpflx on the normal predictor states (Godunov_3D.cpp:180-216);
-// the boundary overrides of Hydro_cmpflx.H:239-282 are written back to the
-// state arrays because the transverse stages read them.
-template <int D>
-__global__ void __launch_bounds__(kBlock)
-k_riemann1(Batch B, HydroConst hc) {
-    BATCH_POINT(ST_R1 + D)
-    const CView q = cview(L, slot_ptr<S_Q>(E), NQC), F = cview(L, slot_ptr<S_F1 + D>(E), NTF);
-    const CView qm = cview(L, slot_ptr<S_QM0 + D>(E), NS), qp = cview(L, slot_ptr<S_QP0 + D>(E), NS);
+// ------------------------------------------------ traces + first fluxes
+// The normal predictor states of direction D and hydro_cmpflx on them
+// (Godunov_3D.cpp:104-216).  A thread traces its cell and owns the cell's
+// low face: the plus state is its own, the minus state and sound speed come
+// from the thread of the cell below through LDS, so that the states are
+// written once and never read back for the first solve.  The boundary
+// overrides of Hydro_cmpflx.H:239-282 stay in the stored states, because
+// the transverse stages read them.
+//
+// What bounds it (256^3, PPM): waiting for loads, half of a wavefront's
+// time; VALU issue is at 51 %, 18.7 GB of traffic at 3.4 TB/s.  So a wave
+// gets the registers to issue its 47 loads at once (3 waves per SIMD:
+// 5.40 ms per step; 4 waves with loads between the arithmetic 6.00 ms, 5
+// and 6 waves spill: 7.7 and 9.4 ms).  The tile of 16 cells along y or z
+// keeps the 5-point stencil in the CU's own cache: separate launches over
+// rows read 19.5 GB where this reads 6.4 GB, and the first solve no longer
+// reads the 18 state values back.  Traces and first solves as six launches
+// took 6.39 ms.  One launch for three directions: at 16^3 the launches and
+// not the work are what is waited for (k_plm_c + k_riemann1 at 16^3: 41 us
+// in 6 launches).
+constexpr int kF1MinWaves = 3;
+#define F1_BOUNDS __launch_bounds__(kBlock, kF1MinWaves)
+constexpr int kF1Slots = NS + 2;  // minus state, sound speed, its floor
+template <int D, int PPM>
+__device__ __forceinline__ void face1_body(const Batch &B, int w, int nw, int has_src,
+                                           const HydroConst &hc, const double *dtp,
+                                           double *sh) {
+    int lblk;
+    const BoxEnt &E = B.tab[batch_box(B, w, nw, lblk)];
+    const Canon L = E.L;
+    const Box g = grow(E.bx, 2);
+    const int t = (int)threadIdx.x;
+    constexpr int step = D == 0 ? 1 : kF1Cols;  // to the thread of the cell below
+    int i = 0, j = 0, k = 0;
+    bool cell, face;
+    if (D == 0) {
+        cell = range_point(range_of(g), (int64_t)lblk * (kBlock - 1) + t, i, j, k);
+        face = cell && t > 0 && i > g.lo[0];
+    } else {
+        const int n0 = g.len(0), across = n0 * g.len(3 - D);
+        const int nm = (across + kF1Cols - 1) / kF1Cols;
+        const int tile = lblk / nm, m = (lblk - tile * nm) * kF1Cols + (t & (kF1Cols - 1));
+        const int row = t / kF1Cols, c = g.lo[D] + tile * (kF1Rows - 1) + row;
+        const int b = m / n0;
+        i = g.lo[0] + m - b * n0;
+        j = D == 1 ? c : g.lo[1] + b;
+        k = D == 1 ? g.lo[2] + b : c;
+        cell = m < across && c <= g.hi[D];
+        face = cell && row > 0;
+    }
+    const CView q = cview(L, slot_ptr<S_Q>(E), NQC);
     const unsigned v0 = L.off(i, j, k), sd = shift<D>(L);
-    double ql[NS], qr[NS];
+    double op[NS];
+    FaceAux a;
+    if (cell) {
+        const double dtdx = *dtp / hc.dx[D];
+        const double fl = cview(L, slot_ptr<S_FLAT>(E), 1).ld(v0, 0);
+        double om[NS];
+        a.c_r = q.ld(v0, SC);
+        a.csml_r = q.ld(v0, SCS);
+        if (PPM)
+            ppm_cell<D>(q, v0, sd, fl, a.c_r, dtdx, hc, op, om);
+        else
+            plm_cell<D>(q, cview(L, slot_ptr<S_SRCQ>(E), NS), has_src, v0, sd, fl, a.c_r, dtdx,
+                        hc, op, om);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) sh[s * kBlock + t] = om[s];
+        sh[NS * kBlock + t] = a.c_r;
+        sh[(NS + 1) * kBlock + t] = a.csml_r;
+    }
+    __syncthreads();
+    if (!face) return;
+    double ql[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) ql[s] = sh[s * kBlock + t - step];
+    a.c_l = sh[NS * kBlock + t - step];
+    a.csml_l = sh[(NS + 1) * kBlock + t - step];
+    a.gam_l = kGamma;
+    a.gam_r = kGamma;
+    const int idx = (D == 0) ? i : ((D == 1) ? j : k);
+    double f[NF], gd[NG];
+    int mut;
+    face_flux(D, idx, hc, ql, op, a, f, gd, &mut);
+    const CView qm = cview(L, slot_ptr<S_QM0 + D>(E), NS), qp = cview(L, slot_ptr<S_QP0 + D>(E), NS);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        ql[s] = qm.ld(v0, s);
-        qr[s] = qp.ld(v0, s);
+        qm.st(v0, s, ql[s]);
+        qp.st(v0, s, op[s]);
     }
-    const FaceAux a = face_aux(q, v0 - sd, v0);
-    const int idx = (D == 0) ? i : ((D == 1) ? j : k);
-    double f[NF], g[NG];
-    int mut;
-    face_flux(D, idx, hc, ql, qr, a, f, g, &mut);
-    if (mut & 1) {
-        qm.st(v0, SR, ql[SR]); qm.st(v0, SP, ql[SP]); qm.st(v0, SE, ql[SE]);
-    }
-    if (mut & 2) {
-        qp.st(v0, SR, qr[SR]); qp.st(v0, SP, qr[SP]); qp.st(v0, SE, qr[SE]);
-    }
-    store_tflux(F, v0, f, g);
+    store_tflux(cview(L, slot_ptr<S_F1 + D>(E), NTF), v0, f, gd);
+}
+
+template <int D>
+__device__ __forceinline__ void face1_ppm(const Batch &B, int w, int nw, int has_src,
+                                          const HydroConst &hc, const double *dtp, double *sh) {
+    face1_body<D, 1>(B, w, nw, has_src, hc, dtp, sh);
+}
+template <int D>
+__device__ __forceinline__ void face1_plm(const Batch &B, int w, int nw, int has_src,
+                                          const HydroConst &hc, const double *dtp, double *sh) {
+    face1_body<D, 0>(B, w, nw, has_src, hc, dtp, sh);
+}
+
+__global__ void F1_BOUNDS
+k_face1_ppm(Batch3 T, HydroConst hc, const double *dtp) {
+    if (T.d[0].halt && *T.d[0].halt) return;  // uniform: the whole block leaves
+    __shared__ double sh[kF1Slots * kBlock];
+    BATCH3_DISPATCH(T, face1_ppm, 0, hc, dtp, sh);
+}
+__global__ void F1_BOUNDS
+k_face1_plm(Batch3 T, int has_src, HydroConst hc, const double *dtp) {
+    if (T.d[0].halt && *T.d[0].halt) return;  // uniform: the whole block leaves
+    __shared__ double sh[kF1Slots * kBlock];
+    BATCH3_DISPATCH(T, face1_plm, has_src, hc, dtp, sh);
 }
 
 // ------------------------------------------------ transdo + Riemann (pairs)
@@ -1415,8 +1480,9 @@ k_update_c(Batch B, HydroConst hc, const double *dtp, int *flags) {
 
 // --------------------------------------------------------------- engine
 // block prefix rows: the stage kinds as tuned, the same without z-march
-// (LaunchCfg linear), then the CTU face kernels of the three directions
-constexpr int kCtuRow0 = 2 * ST_COUNT, kBlkRows = 2 * ST_COUNT + 3;
+// (LaunchCfg linear), then the CTU face kernels and the trace + first-flux
+// kernels of the three directions
+constexpr int kCtuRow0 = 2 * ST_COUNT, kFace1Row0 = kCtuRow0 + 3, kBlkRows = kFace1Row0 + 3;
 
 Tuning default_tuning() {
     Tuning t;
@@ -1557,14 +1623,16 @@ int FusedEngine::build_tables() {
     blk_host_.assign((size_t)kBlkRows * (n + 1), 0);
     for (int k = 0; k < kBlkRows; ++k) {
         int *row = &blk_host_[(size_t)k * (n + 1)];
-        const bool ctu = k >= kCtuRow0;
-        const int kind = ctu ? ST_T2 + (k - kCtuRow0) : k % ST_COUNT;
+        const bool face1 = k >= kFace1Row0, ctu = !face1 && k >= kCtuRow0;
+        const int kind = face1 ? ST_R1 + (k - kFace1Row0)
+                       : ctu ? ST_T2 + (k - kCtuRow0) : k % ST_COUNT;
         const int zm = k < ST_COUNT ? tune_.zm[kind] : 0;
         for (int p = 0; p < n; ++p) {
             const int *l = tune_.tile[kind];
             const Box sb = stage_box(kind, boxes_[order_[p]]);
             const int64_t nb =
-                ctu ? ctu_blocks(sb, tune_.ctu_planes, kind == ST_T2)
+                face1 ? face1_blocks(boxes_[order_[p]], k - kFace1Row0)
+                : ctu ? ctu_blocks(sb, tune_.ctu_planes, kind == ST_T2)
                     : batch_blocks(sb, tune_.block[kind], l[0], l[1], l[2], zm);
             if ((int64_t)row[p] + nb > 0x7fffffff) {
                 set_error("stage grid exceeds 2^31 blocks");
@@ -1594,9 +1662,8 @@ int FusedEngine::enable_adjoint() {
     return build_tables();
 }
 
-LaunchCfg FusedEngine::cfg(int kind, int b, int parity, bool linear) const {
+LaunchCfg FusedEngine::cfg_row(int rk, int b, int parity) const {
     const int n = (int)boxes_.size();
-    const int rk = kind + (linear ? ST_COUNT : 0);
     const int *row = &blk_host_[(size_t)rk * (n + 1)];
     LaunchCfg c;
     c.B.tab = tab_[parity];
@@ -1610,14 +1677,45 @@ LaunchCfg FusedEngine::cfg(int kind, int b, int parity, bool linear) const {
         c.B.first = row[p];
         c.grid = (unsigned)(row[p + 1] - row[p]);
     }
-    c.block = tune_.block[kind];
+    c.block = kBlock;
     c.B.halt = halt_;
+    c.B.lx = -1;
+    c.B.ly = c.B.lz = 0;
+    c.B.xk = 0;
+    c.B.zm = 0;
+    return c;
+}
+
+LaunchCfg FusedEngine::cfg(int kind, int b, int parity, bool linear) const {
+    LaunchCfg c = cfg_row(kind + (linear ? ST_COUNT : 0), b, parity);
+    c.block = tune_.block[kind];
     c.B.lx = tune_.tile[kind][0];
     c.B.ly = tune_.tile[kind][1];
     c.B.lz = tune_.tile[kind][2];
     c.B.xk = tune_.xcd[kind];
     c.B.zm = linear ? 0 : tune_.zm[kind];
     return c;
+}
+
+LaunchCfg FusedEngine::cfg_face1(int d, int b, int parity) const {
+    LaunchCfg c = cfg_row(kFace1Row0 + d, b, parity);
+    c.B.xk = tune_.xcd[ST_R1 + d];
+    return c;
+}
+
+template <typename K, typename... A>
+void FusedEngine::launch3(const char *name, Prof *prof, K kern, const LaunchCfg c[3],
+                          hipStream_t st, A... args) {
+    Batch3 T;
+    int n = 0;
+    for (int d = 0; d < 3; ++d) {
+        T.d[d] = c[d].B;
+        n += (int)c[d].grid;
+        T.end[d] = n;
+    }
+    if (n == 0) return;
+    Region reg(prof, name, st);
+    hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(c[0].block), 0, st, T, args...);
 }
 
 template <typename K, typename... A>
@@ -1630,25 +1728,8 @@ void FusedEngine::launch(const char *name, Prof *prof, K kern, int kind, int b, 
 }
 
 LaunchCfg FusedEngine::cfg_ctu(int d, int b, int parity) const {
-    const int n = (int)boxes_.size();
-    const int rk = kCtuRow0 + d;
-    const int *row = &blk_host_[(size_t)rk * (n + 1)];
-    LaunchCfg c;
-    c.B.tab = tab_[parity];
-    c.B.blk = blk_dev_ + (size_t)rk * (n + 1);
-    c.B.nbox = n;
-    if (b < 0) {
-        c.B.first = 0;
-        c.grid = (unsigned)row[n];
-    } else {
-        const int p = pos_[b];
-        c.B.first = row[p];
-        c.grid = (unsigned)(row[p + 1] - row[p]);
-    }
+    LaunchCfg c = cfg_row(kCtuRow0 + d, b, parity);
     c.block = kCtuBlock;
-    c.B.halt = halt_;
-    c.B.lx = -1;
-    c.B.ly = c.B.lz = 0;
     c.B.xk = tune_.xcd[ST_T2 + d];
     c.B.zm = tune_.ctu_planes;
     return c;
@@ -1677,18 +1758,14 @@ int FusedEngine::hydro(int b, int parity, bool have_prim, const DevFab *sb_tab,
     else
         launch("flatten", prof, k_flat_c<false>, ST_G2, b, parity, st, hc.use_flattening, qgrow,
                sb_tab, hc, status);
-    if (hc.ppm_type == 1) {
-        launch("trace_ppm", prof, k_ppm_c<0>, ST_G2, b, parity, st, hc, dtp);
-        launch("trace_ppm", prof, k_ppm_c<1>, ST_G2, b, parity, st, hc, dtp);
-        launch("trace_ppm", prof, k_ppm_c<2>, ST_G2, b, parity, st, hc, dtp);
-    } else {
-        launch("trace_plm", prof, k_plm_c<0>, ST_G2, b, parity, st, has_src, hc, dtp);
-        launch("trace_plm", prof, k_plm_c<1>, ST_G2, b, parity, st, has_src, hc, dtp);
-        launch("trace_plm", prof, k_plm_c<2>, ST_G2, b, parity, st, has_src, hc, dtp);
+    {
+        const LaunchCfg c[3] = {cfg_face1(0, b, parity), cfg_face1(1, b, parity),
+                                cfg_face1(2, b, parity)};
+        if (hc.ppm_type == 1)
+            launch3("trace_riemann", prof, k_face1_ppm, c, st, hc, dtp);
+        else
+            launch3("trace_riemann", prof, k_face1_plm, c, st, has_src, hc, dtp);
     }
-    launch("riemann_normal", prof, k_riemann1<0>, ST_R1 + 0, b, parity, st, hc);
-    launch("riemann_normal", prof, k_riemann1<1>, ST_R1 + 1, b, parity, st, hc);
-    launch("riemann_normal", prof, k_riemann1<2>, ST_R1 + 2, b, parity, st, hc);
     // the adjoint's recompute (no_update) reads the transdo fluxes
     const bool ctu = tune_.ctu && !no_update;
     if (ctu) {
@@ -1815,18 +1892,20 @@ int fused_umdrv(const UmdrvArgs &A, double *scratch, hipStream_t st) {
     const int has_src = A.has_src;
     launch_one(k_flat_c<false>, ST_G2, bx, B, st, hc.use_flattening, (int)CAMR_NGROW,
                (const DevFab *)nullptr, hc, (int *)nullptr);
-    if (hc.ppm_type == 1) {
-        launch_one(k_ppm_c<0>, ST_G2, bx, B, st, hc, dtp);
-        launch_one(k_ppm_c<1>, ST_G2, bx, B, st, hc, dtp);
-        launch_one(k_ppm_c<2>, ST_G2, bx, B, st, hc, dtp);
-    } else {
-        launch_one(k_plm_c<0>, ST_G2, bx, B, st, has_src, hc, dtp);
-        launch_one(k_plm_c<1>, ST_G2, bx, B, st, has_src, hc, dtp);
-        launch_one(k_plm_c<2>, ST_G2, bx, B, st, has_src, hc, dtp);
+    {
+        Batch3 T;
+        int n = 0;
+        for (int d = 0; d < 3; ++d) {
+            T.d[d] = B;
+            n += (int)face1_blocks(bx, d);
+            T.end[d] = n;
+        }
+        if (hc.ppm_type == 1)
+            hipLaunchKernelGGL(k_face1_ppm, dim3((unsigned)n), dim3(kBlock), 0, st, T, hc, dtp);
+        else
+            hipLaunchKernelGGL(k_face1_plm, dim3((unsigned)n), dim3(kBlock), 0, st, T, has_src, hc,
+                               dtp);
     }
-    launch_one(k_riemann1<0>, ST_R1 + 0, bx, B, st, hc);
-    launch_one(k_riemann1<1>, ST_R1 + 1, bx, B, st, hc);
-    launch_one(k_riemann1<2>, ST_R1 + 2, bx, B, st, hc);
     launch_one(k_trans1_x, ST_T1 + 0, bx, B, st, hc, dtp);
     launch_one(k_trans1<1>, ST_T1 + 1, bx, B, st, hc, dtp);
     launch_one(k_trans1<2>, ST_T1 + 2, bx, B, st, hc, dtp);

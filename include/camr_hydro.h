@@ -399,8 +399,10 @@ int camr_level_get_tuning(camr_level *L, int32_t block[CAMR_NSTAGE], int32_t *or
  * {64, 128, 256} (that product becomes the stage's block size), or (0, 0, 0)
  * for blocks of consecutive points in x-fastest order.  A tile keeps the
  * y and z stencil neighbours of a block's points inside the block.
- * camr_level_set_tuning resets every stage to (0, 0, 0).  No reference
- * counterpart: set by the autotuner. */
+ * camr_level_set_tuning resets every stage to (0, 0, 0).  The first-flux
+ * faces, solved where their states are traced, keep a shape of their own
+ * and take only the XCD chunk.  No reference counterpart: set by the
+ * autotuner. */
 int camr_level_set_tiles(camr_level *L, const int32_t tile[3 * CAMR_NSTAGE]);
 int camr_level_get_tiles(camr_level *L, int32_t tile[3 * CAMR_NSTAGE]);
 /* XCD chunk of each stage range: 0 keeps the hardware's round-robin of
