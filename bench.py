@@ -56,6 +56,7 @@ NS_MOL_READ, NF_MOL_WRITE = 23, 12
 # FETCH_SIZE scaled by 1.9692, WRITE_SIZE by 0.9961, the factors an
 # 8-byte-lane copy of 1 GiB reads back).  Reported only for that engine and size.
 MEASURED_TRAFFIC = {("fused", 256, "transverse_2"): 10447411888,
+                    ("fused", 256, "trace_riemann"): 18670000000,
                     ("fused", 256, "transverse_ctu"): 28527364887}
 
 # Executed FP64 work of one PPM cell-update (ADD, MUL, TRANS = 1, FMA = 2 per
@@ -70,8 +71,8 @@ FP64_EXECUTED_PER_CELL_UPDATE = 10069
 # (`python oracle/count_ops.py --n 256`, profiles/fp64_opcount_256cube_ppm.md).
 # Keys are the profiler regions of the fused engine; a face stage's count
 # covers its three launches (one per direction).
-ALGO_FLOP = {"fill_clean_prim": 169.0, "flatten": 59.3,
-             "trace_riemann": 3501.9 + 300.6, "transverse_1": 1285.1, "divu": 30.4,
+ALGO_FLOP = {"fill_clean_prim": 169.0, "flatten_divu": 59.3 + 30.4,
+             "trace_riemann": 3501.9 + 300.6, "transverse_1": 1285.1,
              "transverse_2": 989.9, "consup_clean_estdt": 111.0 + 129.0}
 ALGO_FLOP_PER_CELL_UPDATE = sum(ALGO_FLOP.values())
 # the CTU face kernels do the work of both transverse stages
@@ -932,9 +933,12 @@ def main() -> int:
     avg_ms = rep["ms"] / rep["count"]
     # algorithmic FP64 operations of one launch of the dominant kernel: its
     # stage's count per cell-update over the launches of that stage per step
-    flop_launch = ALGO_FLOP.get(kern, 0.0) * n ** 3 / LAUNCHES_PER_STEP.get(kern, 1)
+    # (small levels run a stage's three directions as one launch)
+    launches = rep["count"] / args.steps
+    flop_launch = ALGO_FLOP.get(kern, 0.0) * n ** 3 / launches
     achieved = flop_launch / (avg_ms * 1e-3) / 1e12
-    algo_bytes = ALGO_DOUBLES.get(kern, 2 * NVAR) * 8 * unit_count(kern, n)
+    algo_bytes = (ALGO_DOUBLES.get(kern, 2 * NVAR) * 8 * unit_count(kern, n)
+                  * LAUNCHES_PER_STEP.get(kern, 1) / launches)
     tiles = L.tiles if args.engine == "fused" else None
     ctu = L.ctu if args.engine == "fused" else None
 

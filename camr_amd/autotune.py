@@ -53,15 +53,14 @@ CANDIDATES = tuple((bs, LINEAR, k) for bs in BLOCKS for k in XCD_CHUNKS) + tuple
 # profiler region name -> stage-range indices (CAMR_NSTAGE order)
 STAGES = {
     "fill_clean_prim": (0,), "prim": (0,),
-    "flatten": (1,),
+    "flatten_divu": (1, 8),  # one launch when the two block sizes agree
     "trace_riemann": (2, 3, 4),  # only the XCD chunk: the stage has its own blocks
     "transverse_1": (5, 6, 7),
-    "divu": (8,),
     "transverse_2": (9, 10, 11),
     "consup": (12,), "clean_estdt": (12,), "consup_clean_estdt": (12,),
 }
 # groups of stage ranges that must share a block size (one profiler name)
-GROUPS = [(0,), (1,), (2, 3, 4), (5, 6, 7), (8,), (9, 10, 11), (12,)]
+GROUPS = [(0,), (1, 8), (2, 3, 4), (5, 6, 7), (9, 10, 11), (12,)]
 
 
 def cache_path() -> str:

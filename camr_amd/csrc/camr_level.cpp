@@ -3482,9 +3482,7 @@ int camr_hydro_umdrv(const camr_box *bx, const camr_array4 *uin, const camr_arra
     double *scr = nullptr;
     CAMR_HIP(hipMallocFromPoolAsync((void **)&scr, (n + 1) * sizeof(double), pool, s));
     if (fused) {
-        A.dtp = scr + n;
-        put_double(scr + n, dt, s);
-        rc = fused_umdrv(A, scr, s);
+        rc = fused_umdrv(A, dt, scr, s);
         if (rc) set_error("kernel launch failed");
     } else {
         rc = umdrv_run(A, scr, n, dt, p->do_mol, s);

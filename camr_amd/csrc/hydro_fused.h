@@ -481,6 +481,7 @@ class FusedEngine {
                  A... args);
     // block-prefix row rk (see kBlkRows), table entry range of box b
     LaunchCfg cfg_row(int rk, int b, int parity) const;
+    bool merge_faces(int kind, int b, int parity, LaunchCfg c[3]) const;
     // grid of the trace + first-flux kernel of direction d
     LaunchCfg cfg_face1(int d, int b, int parity) const;
     // grid of the CTU face kernel of direction d
@@ -519,6 +520,6 @@ Tuning default_tuning();
 struct UmdrvArgs;
 bool fused_umdrv_applies(const UmdrvArgs &A, int do_mol);
 size_t fused_umdrv_scratch_doubles(const Box &bx);
-int fused_umdrv(const UmdrvArgs &A, double *scratch, hipStream_t st);
+int fused_umdrv(const UmdrvArgs &A, double dt, double *scratch, hipStream_t st);
 
 } // namespace camr

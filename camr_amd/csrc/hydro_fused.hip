@@ -4,7 +4,7 @@
 // Hydro_umdrv.cpp:11-93), re-organised around faces so that no transverse
 // or final interface state ever goes to HBM:
 //   k_prim_c    U -> compact primitives (rho u v w p rhoe Y0..2 c csml)
-//   k_flat_c    shock flattening coefficient
+//   k_flat_divu shock flattening coefficient, nodal divergence
 //   k_face1     normal predictor states, face-indexed, and the first fluxes
 //               (with the reference's boundary-face mutation)
 //   k_trans1<D> per D-face: the two transdo states of each side are formed
@@ -149,10 +149,10 @@ __device__ __forceinline__ double flat_dir(const CView &q, const Canon &L, unsig
 // WIDE: q's box is grow(bx, qgrow) with qgrow > 4 (points beyond the
 // canonical primitives from sb_tab); else grow(bx, 4)
 template <bool WIDE>
-__global__ void __launch_bounds__(kBlock)
-k_flat_c(Batch B, int use_flattening, int qgrow, const DevFab *sb_tab, HydroConst hc,
-         int *status) {
-    BATCH_POINT(ST_G2)
+__device__ __forceinline__ void flat_point(const Batch &B, int w, int nw, int use_flattening,
+                                           int qgrow, const DevFab *sb_tab,
+                                           const HydroConst &hc, int *status) {
+    BATCH_POINT_AT(ST_G2, w, nw)
     const CView q = cview(L, slot_ptr<S_Q>(E), NQC), flat = cview(L, slot_ptr<S_FLAT>(E), 1);
     const Arr u = WIDE ? sb_tab[E.id].a : Arr{};
     const unsigned v0 = L.off(i, j, k);
@@ -163,6 +163,26 @@ k_flat_c(Batch B, int use_flattening, int qgrow, const DevFab *sb_tab, HydroCons
         f = vmin(f, flat_dir<2, WIDE>(q, L, v0, i, j, k, E.bx, qgrow, u, hc, status));
     }
     flat.st(v0, 0, f);
+}
+
+__device__ __forceinline__ void divu_point(const Batch &B, int w, int nw, const HydroConst &hc) {
+    BATCH_POINT_AT(ST_DIVU, w, nw)
+    // compact q has u, v, w in the same slots as QU, QV, QW
+    const CView q = cview(L, slot_ptr<S_Q>(E), NQC), divu = cview(L, slot_ptr<S_DIVU>(E), 1);
+    divu.st(L.off(i, j, k), 0, divu_node(q, i, j, k, hc));
+}
+
+// The flattening of grow(bx, 2) (T.d[0]) and the nodal divergence (T.d[1]),
+// which both read the primitives alone: one launch instead of two.
+template <bool WIDE>
+__global__ void __launch_bounds__(kBlock)
+k_flat_divu(Batch3 T, int use_flattening, int qgrow, const DevFab *sb_tab, HydroConst hc,
+            int *status) {
+    const int w = (int)blockIdx.x;
+    if (w < T.end[0])
+        flat_point<WIDE>(T.d[0], w, T.end[0], use_flattening, qgrow, sb_tab, hc, status);
+    else
+        divu_point(T.d[1], w - T.end[0], T.end[1] - T.end[0], hc);
 }
 
 // ------------------------------------------------------------ traces
@@ -433,9 +453,9 @@ __device__ __forceinline__ void trans1_pair(unsigned v0, const Canon &L, const d
 }
 
 template <int D>
-__global__ void TRANS_BOUNDS
-k_trans1(Batch B, HydroConst hc, const double *dtp) {
-    BATCH_POINT(ST_T1 + D)
+__device__ __forceinline__ void trans1_point(const Batch &B, int w, int nw, const HydroConst &hc,
+                                             const double *dtp) {
+    BATCH_POINT_AT(ST_T1 + D, w, nw)
     constexpr int T0 = (D == 0) ? 1 : 0;
     constexpr int T1 = (D == 2) ? 1 : 2;
     const double cda = 1.0 / 3.0 * *dtp / hc.dx[T0];
@@ -474,15 +494,32 @@ __device__ __forceinline__ void trans2_diff(unsigned v, const Canon &L, const CV
     trans_diff_two(fal, far_, gal, gar, fbl, fbr, gbl, gbr, ca, cb, kGamma, t);
 }
 
+// The final flux of the D-face (i,j,k) at offset v0: into the canonical
+// array, or (OUT) its NVAR components into the caller's array flx and only
+// the Godunov (u, p) into the canonical one.
+template <int D, int OUT>
+__device__ __forceinline__ void store_final(const BoxEnt &E, const Canon &L, unsigned v0, int i,
+                                            int j, int k, const double *fu, const double *g,
+                                            const Arr &flx) {
+    const CView c = cview(L, slot_ptr<S_FLX + D>(E), NXF);
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) {
+        if (OUT) flx(i, j, k, n) = fu[n];
+        else c.st(v0, n, fu[n]);
+    }
+    c.st(v0, XGU, g[GUN]);
+    c.st(v0, XGP, g[GP]);
+}
+
 // ---------------------------------- transdd + final Riemann + adjust_fluxes
 // D-face f: plus state from transdd at cell f, minus state from transdd at
 // cell f-e_D (Godunov_utils_3D.H:245-482); then hydro_cmpflx, then
 // hydro_artif_visc / hydro_norm_spec_flx / hydro_ext_flx
 // (Hydro_adjust_fluxes.cpp:13-44).
-template <int D, int HAS_SRC>
-__global__ void TRANS_BOUNDS
-k_trans2(Batch B, HydroConst hc, const double *dtp) {
-    BATCH_POINT(ST_T2 + D)
+template <int D, int HAS_SRC, int OUT>
+__device__ __forceinline__ void trans2_point(const Batch &B, int w, int nw, const HydroConst &hc,
+                                             const double *dtp, const Arr &flx) {
+    BATCH_POINT_AT(ST_T2 + D, w, nw)
     constexpr int T0 = (D == 0) ? 1 : 0;
     constexpr int T1 = (D == 2) ? 1 : 2;
     const double dt = *dtp;
@@ -531,11 +568,7 @@ k_trans2(Batch B, HydroConst hc, const double *dtp) {
     for (int s = 0; s < NSPEC; ++s) fu[UFS + s] = f[FY + s];
     adjust_face<D>(fu, cview(L, slot_ptr<S_DIVU>(E), 1), cview(L, slot_ptr<S_U>(E), NVAR), i, j,
                    k, area, hc);
-    const CView flx = cview(L, slot_ptr<S_FLX + D>(E), NXF);
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n) flx.st(v0, n, fu[n]);
-    flx.st(v0, XGU, g[GUN]);
-    flx.st(v0, XGP, g[GP]);
+    store_final<D, OUT>(E, L, v0, i, j, k, fu, g, flx);
 }
 
 // ------------------------------------------------ z-marching z-face kernels
@@ -779,9 +812,9 @@ __device__ __forceinline__ void lane_up_td2(const TransDiff &a, TransDiff &b) {
     b.pnew = lane_up(a.pnew);
 }
 
-__global__ void TRANS_BOUNDS
-k_trans1_x(Batch B, HydroConst hc, const double *dtp) {
-    BATCH_POINT(ST_T1 + 0)
+__device__ __forceinline__ void trans1_x_point(const Batch &B, int w, int nw,
+                                               const HydroConst &hc, const double *dtp) {
+    BATCH_POINT_AT(ST_T1 + 0, w, nw)
     const double cda = 1.0 / 3.0 * *dtp / hc.dx[1];
     const double cdb = 1.0 / 3.0 * *dtp / hc.dx[2];
     const CView q = cview(L, slot_ptr<S_Q>(E), NQC);
@@ -834,10 +867,11 @@ k_trans1_x(Batch B, HydroConst hc, const double *dtp) {
     }
 }
 
-template <int HAS_SRC>
-__global__ void TRANS_BOUNDS
-k_trans2_x(Batch B, HydroConst hc, const double *dtp) {
-    BATCH_POINT(ST_T2 + 0)
+template <int HAS_SRC, int OUT>
+__device__ __forceinline__ void trans2_x_point(const Batch &B, int w, int nw,
+                                               const HydroConst &hc, const double *dtp,
+                                               const Arr &flx) {
+    BATCH_POINT_AT(ST_T2 + 0, w, nw)
     const double dt = *dtp;
     const double hdt = 0.5 * dt;
     const double ca = 0.5 * dt / hc.dx[1], cb = 0.5 * dt / hc.dx[2];
@@ -906,11 +940,68 @@ k_trans2_x(Batch B, HydroConst hc, const double *dtp) {
     d4[2] = dv.ld(v0 + sz, 0);
     d4[3] = dv.ld(v0 + sy + sz, 0);
     adjust_face_vals<0>(fu, d4, up, um, i, area, hc);
-    const CView flx = cview(L, slot_ptr<S_FLX + 0>(E), NXF);
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n) flx.st(v0, n, fu[n]);
-    flx.st(v0, XGU, g[GUN]);
-    flx.st(v0, XGP, g[GP]);
+    store_final<0, OUT>(E, L, v0, i, j, k, fu, g, flx);
+}
+
+// ------------------------------------------------ transverse launches
+// One launch per direction: each direction's registers and, for z, the
+// marching kernels above; what large levels run.
+template <int D>
+__global__ void TRANS_BOUNDS
+k_trans1(Batch B, HydroConst hc, const double *dtp) {
+    if (D == 0) trans1_x_point(B, (int)blockIdx.x, (int)gridDim.x, hc, dtp);
+    else trans1_point<D>(B, (int)blockIdx.x, (int)gridDim.x, hc, dtp);
+}
+template <int D, int HAS_SRC>
+__global__ void TRANS_BOUNDS
+k_trans2(Batch B, HydroConst hc, const double *dtp) {
+    if (D == 0) trans2_x_point<HAS_SRC, 0>(B, (int)blockIdx.x, (int)gridDim.x, hc, dtp, Arr{});
+    else trans2_point<D, HAS_SRC, 0>(B, (int)blockIdx.x, (int)gridDim.x, hc, dtp, Arr{});
+}
+
+// All three directions in one launch, for levels whose launches are short
+// (see kMergeBlocks).
+template <int D>
+__device__ __forceinline__ void trans1_any(const Batch &B, int w, int nw, const HydroConst &hc,
+                                           const double *dtp) {
+    if (D == 0) trans1_x_point(B, w, nw, hc, dtp);
+    else trans1_point<D>(B, w, nw, hc, dtp);
+}
+struct FluxOut {
+    Arr f[3];
+};
+template <int D, int HAS_SRC, int OUT>
+__device__ __forceinline__ void trans2_dir(const Batch &B, int w, int nw, const HydroConst &hc,
+                                           const double *dtp, const FluxOut &o) {
+    if (D == 0) trans2_x_point<HAS_SRC, OUT>(B, w, nw, hc, dtp, o.f[0]);
+    else trans2_point<D, HAS_SRC, OUT>(B, w, nw, hc, dtp, o.f[D]);
+}
+template <int HAS_SRC, int OUT>
+struct Trans2 {
+    template <int D>
+    static __device__ __forceinline__ void any(const Batch &B, int w, int nw,
+                                               const HydroConst &hc, const double *dtp,
+                                               const FluxOut &o) {
+        trans2_dir<D, HAS_SRC, OUT>(B, w, nw, hc, dtp, o);
+    }
+};
+// (the registers of the widest direction: 3 waves per SIMD)
+__global__ void TRANS_BOUNDS
+k_trans1_all(Batch3 T, HydroConst hc, const double *dtp) {
+    BATCH3_DISPATCH(T, trans1_any, hc, dtp);
+}
+template <int HAS_SRC>
+__global__ void TRANS_BOUNDS
+k_trans2_all(Batch3 T, HydroConst hc, const double *dtp) {
+    typedef Trans2<HAS_SRC, 0> K;
+    BATCH3_DISPATCH(T, K::template any, hc, dtp, FluxOut{});
+}
+// the one-box route: the fluxes go straight into the caller's arrays
+template <int HAS_SRC>
+__global__ void TRANS_BOUNDS
+k_trans2_box(Batch3 T, HydroConst hc, const double *dtp, FluxOut o) {
+    typedef Trans2<HAS_SRC, 1> K;
+    BATCH3_DISPATCH(T, K::template any, hc, dtp, o);
 }
 
 // ------------------------------------------------ LDS-staged CTU face kernels
@@ -1344,6 +1435,7 @@ __global__ void CTU_BOUNDS k_ctu_y(Batch B, HydroConst hc, const double *dtp) {
 // The table of a one-box launch: its entry and a block prefix of {0}.
 struct OneBox {
     BoxEnt e;
+    double dt;
     int blk0;
 };
 __global__ void k_put_onebox(OneBox *dst, OneBox v) {
@@ -1385,22 +1477,11 @@ k_box_in(Batch B, Arr q, Arr qa, Arr srcq, int has_src, Arr uin, Box ubox) {
     }
 }
 
-// The final d-fluxes of the canonical array into the caller's flx[d].
-template <int D>
-__global__ void __launch_bounds__(kBlock)
-k_box_flux_out(Batch B, Arr flx) {
-    BATCH_POINT(ST_T2 + D)
-    const CView f = cview(L, slot_ptr<S_FLX + D>(E), NXF);
-    const unsigned v0 = L.off(i, j, k);
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n) flx(i, j, k, n) = f.ld(v0, n);
-}
-
 // hydro_pdivu (Hydro_utils_K.H:175-202) and hydro_update (:239-257) into
 // dsdt (+=), in the operation order of the staged k_update with the
 // uniform-grid area and volume.
 __global__ void __launch_bounds__(kBlock)
-k_box_update(Batch B, Arr dsdt, double ac0, double ac1, double ac2, double volc) {
+k_box_update(Batch B, Arr dsdt, FluxOut o, double ac0, double ac1, double ac2, double volc) {
     BATCH_POINT(ST_VALID)
     const CView f0 = cview(L, slot_ptr<S_FLX + 0>(E), NXF), f1 = cview(L, slot_ptr<S_FLX + 1>(E), NXF),
                 f2 = cview(L, slot_ptr<S_FLX + 2>(E), NXF);
@@ -1414,8 +1495,8 @@ k_box_update(Batch B, Arr dsdt, double ac0, double ac1, double ac2, double volc)
     const double volinv = 1.0 / volc;
 #pragma unroll
     for (int n = 0; n < NVAR; ++n) {
-        dsdt(i, j, k, n) += (f0.ld(v0, n) - f0.ld(v0 + sx, n) + f1.ld(v0, n) - f1.ld(v0 + sy, n) +
-                             f2.ld(v0, n) - f2.ld(v0 + sz, n)) *
+        dsdt(i, j, k, n) += (o.f[0](i, j, k, n) - o.f[0](i + 1, j, k, n) + o.f[1](i, j, k, n) -
+                             o.f[1](i, j + 1, k, n) + o.f[2](i, j, k, n) - o.f[2](i, j, k + 1, n)) *
                             volinv;
     }
     dsdt(i, j, k, UEINT) -= pdivu;
@@ -1448,14 +1529,6 @@ k_dsdt_c(Batch B, const DevFab *dsdt_tab, double ac0, double ac1, double ac2, do
     }
 }
 
-__global__ void __launch_bounds__(kBlock)
-k_divu_c(Batch B, HydroConst hc) {
-    BATCH_POINT(ST_DIVU)
-    // compact q has u, v, w in the same slots as QU, QV, QW
-    const CView q = cview(L, slot_ptr<S_Q>(E), NQC), divu = cview(L, slot_ptr<S_DIVU>(E), 1);
-    divu.st(L.off(i, j, k), 0, divu_node(q, i, j, k, hc));
-}
-
 // ------------------------------------------------------------ update
 // hydro_pdivu (Hydro_utils_K.H:175-202), hydro_update (:239-257) on a zeroed
 // dS/dt (CAMR_construct_hydro_source.cpp:14), then the Saxpy of
@@ -1482,6 +1555,16 @@ k_update_c(Batch B, HydroConst hc, const double *dtp, int *flags) {
 // block prefix rows: the stage kinds as tuned, the same without z-march
 // (LaunchCfg linear), then the CTU face kernels and the trace + first-flux
 // kernels of the three directions
+
+// The transverse stages' three directions run as one launch up to this many
+// blocks.  Measured, one launch against three per stage (us per step or
+// call): 256x4x4 PLM 121 against 162, 32^3 level 152 / 176, 64^3 455 / 493,
+// 97x83x61 995 / 1018, 42 refined boxes of 8..32 5250 / 5408 (four steps),
+// 128^3 2861 / 2885, 160^3 (5.0e4 blocks) 5356 / 5357, 256^3 (2.0e5)
+// 21214 / 20786: launches and last waves cost the small ones, while a large
+// one gains more from the z-marching kernels and from registers sized for
+// one direction.
+constexpr int64_t kMergeBlocks = 49152;
 constexpr int kCtuRow0 = 2 * ST_COUNT, kFace1Row0 = kCtuRow0 + 3, kBlkRows = kFace1Row0 + 3;
 
 Tuning default_tuning() {
@@ -1697,6 +1780,18 @@ LaunchCfg FusedEngine::cfg(int kind, int b, int parity, bool linear) const {
     return c;
 }
 
+// The three directions of a transverse stage as one launch: for linear and
+// tiled blocks of one size, up to kMergeBlocks blocks.
+bool FusedEngine::merge_faces(int kind, int b, int parity, LaunchCfg c[3]) const {
+    int64_t n = 0;
+    for (int d = 0; d < 3; ++d) {
+        c[d] = cfg(kind + d, b, parity, true);
+        if (c[d].block != c[0].block) return false;
+        n += c[d].grid;
+    }
+    return n <= kMergeBlocks;
+}
+
 LaunchCfg FusedEngine::cfg_face1(int d, int b, int parity) const {
     LaunchCfg c = cfg_row(kFace1Row0 + d, b, parity);
     c.B.xk = tune_.xcd[ST_R1 + d];
@@ -1707,15 +1802,16 @@ template <typename K, typename... A>
 void FusedEngine::launch3(const char *name, Prof *prof, K kern, const LaunchCfg c[3],
                           hipStream_t st, A... args) {
     Batch3 T;
-    int n = 0;
+    int n = 0, block = kBlock;
     for (int d = 0; d < 3; ++d) {
         T.d[d] = c[d].B;
         n += (int)c[d].grid;
         T.end[d] = n;
+        if (c[d].grid) block = c[d].block;
     }
     if (n == 0) return;
     Region reg(prof, name, st);
-    hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(c[0].block), 0, st, T, args...);
+    hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(block), 0, st, T, args...);
 }
 
 template <typename K, typename... A>
@@ -1752,12 +1848,20 @@ int FusedEngine::hydro(int b, int parity, bool have_prim, const DevFab *sb_tab,
         launch("prim", prof, k_prim_c, ST_G4, b, parity, st, sb_tab, src_tab, has_src, hc, status);
     // q beyond the canonical grow(bx, 4) comes from sb_tab (given with !have_prim)
     const int qgrow = (!have_prim && sb_tab) ? qgrow_ : CAMR_NGROW;
-    if (qgrow > CAMR_NGROW)
-        launch("flatten", prof, k_flat_c<true>, ST_G2, b, parity, st, hc.use_flattening, qgrow,
-               sb_tab, hc, status);
-    else
-        launch("flatten", prof, k_flat_c<false>, ST_G2, b, parity, st, hc.use_flattening, qgrow,
-               sb_tab, hc, status);
+    {
+        const LaunchCfg f = cfg(ST_G2, b, parity), v = cfg(ST_DIVU, b, parity), none{};
+        const LaunchCfg both[3] = {f, v, none}, one[3] = {f, none, none}, two[3] = {none, v, none};
+        const bool split = f.block != v.block;  // tuned to different block sizes
+        for (const LaunchCfg *c : {split ? one : both, split ? two : (const LaunchCfg *)nullptr}) {
+            if (!c) continue;
+            if (qgrow > CAMR_NGROW)
+                launch3("flatten_divu", prof, k_flat_divu<true>, c, st, hc.use_flattening, qgrow,
+                        sb_tab, hc, status);
+            else
+                launch3("flatten_divu", prof, k_flat_divu<false>, c, st, hc.use_flattening, qgrow,
+                        sb_tab, hc, status);
+        }
+    }
     {
         const LaunchCfg c[3] = {cfg_face1(0, b, parity), cfg_face1(1, b, parity),
                                 cfg_face1(2, b, parity)};
@@ -1769,7 +1873,6 @@ int FusedEngine::hydro(int b, int parity, bool have_prim, const DevFab *sb_tab,
     // the adjoint's recompute (no_update) reads the transdo fluxes
     const bool ctu = tune_.ctu && !no_update;
     if (ctu) {
-        launch("divu", prof, k_divu_c, ST_DIVU, b, parity, st, hc);
         if (has_src) {
             launch_ctu("transverse_ctu", prof, k_ctu_x<1>, 0, b, parity, st, hc, dtp);
             launch_ctu("transverse_ctu", prof, k_ctu_y<1>, 1, b, parity, st, hc, dtp);
@@ -1780,23 +1883,30 @@ int FusedEngine::hydro(int b, int parity, bool have_prim, const DevFab *sb_tab,
             launch_ctu("transverse_ctu", prof, k_ctu_z<0>, 2, b, parity, st, hc, dtp);
         }
     } else {
-        launch("transverse_1", prof, k_trans1_x, ST_T1 + 0, b, parity, st, hc, dtp);
-        launch("transverse_1", prof, k_trans1<1>, ST_T1 + 1, b, parity, st, hc, dtp);
-        if (tune_.zm[ST_T1 + 2] > 0)
-            launch("transverse_1", prof, k_trans1_zm, ST_T1 + 2, b, parity, st, hc, dtp);
-        else
-            launch("transverse_1", prof, k_trans1<2>, ST_T1 + 2, b, parity, st, hc, dtp);
-        launch("divu", prof, k_divu_c, ST_DIVU, b, parity, st, hc);
+        LaunchCfg c[3];
+        if (merge_faces(ST_T1, b, parity, c)) {
+            launch3("transverse_1", prof, k_trans1_all, c, st, hc, dtp);
+        } else {
+            launch("transverse_1", prof, k_trans1<0>, ST_T1 + 0, b, parity, st, hc, dtp);
+            launch("transverse_1", prof, k_trans1<1>, ST_T1 + 1, b, parity, st, hc, dtp);
+            if (tune_.zm[ST_T1 + 2] > 0)
+                launch("transverse_1", prof, k_trans1_zm, ST_T1 + 2, b, parity, st, hc, dtp);
+            else
+                launch("transverse_1", prof, k_trans1<2>, ST_T1 + 2, b, parity, st, hc, dtp);
+        }
         const bool zm2 = tune_.zm[ST_T2 + 2] > 0;
-        if (has_src) {
-            launch("transverse_2", prof, k_trans2_x<1>, ST_T2 + 0, b, parity, st, hc, dtp);
+        if (merge_faces(ST_T2, b, parity, c)) {
+            if (has_src) launch3("transverse_2", prof, k_trans2_all<1>, c, st, hc, dtp);
+            else launch3("transverse_2", prof, k_trans2_all<0>, c, st, hc, dtp);
+        } else if (has_src) {
+            launch("transverse_2", prof, k_trans2<0, 1>, ST_T2 + 0, b, parity, st, hc, dtp);
             launch("transverse_2", prof, k_trans2<1, 1>, ST_T2 + 1, b, parity, st, hc, dtp);
             if (zm2)
                 launch("transverse_2", prof, k_trans2_zm<1>, ST_T2 + 2, b, parity, st, hc, dtp);
             else
                 launch("transverse_2", prof, k_trans2<2, 1>, ST_T2 + 2, b, parity, st, hc, dtp);
         } else {
-            launch("transverse_2", prof, k_trans2_x<0>, ST_T2 + 0, b, parity, st, hc, dtp);
+            launch("transverse_2", prof, k_trans2<0, 0>, ST_T2 + 0, b, parity, st, hc, dtp);
             launch("transverse_2", prof, k_trans2<1, 0>, ST_T2 + 1, b, parity, st, hc, dtp);
             if (zm2)
                 launch("transverse_2", prof, k_trans2_zm<0>, ST_T2 + 2, b, parity, st, hc, dtp);
@@ -1863,7 +1973,7 @@ size_t fused_umdrv_scratch_doubles(const Box &bx) {
     return kOneBoxHeader + FusedEngine::scratch_doubles(bx);
 }
 
-int fused_umdrv(const UmdrvArgs &A, double *scratch, hipStream_t st) {
+int fused_umdrv(const UmdrvArgs &A, double dt, double *scratch, hipStream_t st) {
     const Box bx = A.bx;
     const HydroConst &hc = A.hc;
     OneBox ob;
@@ -1873,6 +1983,7 @@ int fused_umdrv(const UmdrvArgs &A, double *scratch, hipStream_t st) {
     ob.e.L = canon_of(bx);
     ob.e.base = scratch + kOneBoxHeader;
     ob.e.abase = nullptr;
+    ob.dt = dt;
     ob.blk0 = 0;
     OneBox *dev = (OneBox *)scratch;
     hipLaunchKernelGGL(k_put_onebox, dim3(1), dim3(64), 0, st, dev, ob);
@@ -1888,41 +1999,36 @@ int fused_umdrv(const UmdrvArgs &A, double *scratch, hipStream_t st) {
     B.zm = 0;
     const Box ubox = grow(bx, 1);
     launch_one(k_box_in, ST_G4, bx, B, st, A.q, A.qaux, A.srcq, A.has_src, A.uin, ubox);
-    const double *dtp = A.dtp;
+    const double *dtp = &dev->dt;
     const int has_src = A.has_src;
-    launch_one(k_flat_c<false>, ST_G2, bx, B, st, hc.use_flattening, (int)CAMR_NGROW,
-               (const DevFab *)nullptr, hc, (int *)nullptr);
-    {
+    auto three = [&](int64_t n0, int64_t n1, int64_t n2) {
         Batch3 T;
-        int n = 0;
-        for (int d = 0; d < 3; ++d) {
-            T.d[d] = B;
-            n += (int)face1_blocks(bx, d);
-            T.end[d] = n;
-        }
-        if (hc.ppm_type == 1)
-            hipLaunchKernelGGL(k_face1_ppm, dim3((unsigned)n), dim3(kBlock), 0, st, T, hc, dtp);
-        else
-            hipLaunchKernelGGL(k_face1_plm, dim3((unsigned)n), dim3(kBlock), 0, st, T, has_src, hc,
-                               dtp);
-    }
-    launch_one(k_trans1_x, ST_T1 + 0, bx, B, st, hc, dtp);
-    launch_one(k_trans1<1>, ST_T1 + 1, bx, B, st, hc, dtp);
-    launch_one(k_trans1<2>, ST_T1 + 2, bx, B, st, hc, dtp);
-    launch_one(k_divu_c, ST_DIVU, bx, B, st, hc);
-    if (has_src) {
-        launch_one(k_trans2_x<1>, ST_T2 + 0, bx, B, st, hc, dtp);
-        launch_one(k_trans2<1, 1>, ST_T2 + 1, bx, B, st, hc, dtp);
-        launch_one(k_trans2<2, 1>, ST_T2 + 2, bx, B, st, hc, dtp);
-    } else {
-        launch_one(k_trans2_x<0>, ST_T2 + 0, bx, B, st, hc, dtp);
-        launch_one(k_trans2<1, 0>, ST_T2 + 1, bx, B, st, hc, dtp);
-        launch_one(k_trans2<2, 0>, ST_T2 + 2, bx, B, st, hc, dtp);
-    }
-    launch_one(k_box_flux_out<0>, ST_T2 + 0, bx, B, st, A.flx[0]);
-    launch_one(k_box_flux_out<1>, ST_T2 + 1, bx, B, st, A.flx[1]);
-    launch_one(k_box_flux_out<2>, ST_T2 + 2, bx, B, st, A.flx[2]);
-    launch_one(k_box_update, ST_VALID, bx, B, st, A.dsdt, A.area_c[0], A.area_c[1], A.area_c[2],
+        for (int d = 0; d < 3; ++d) T.d[d] = B;
+        T.end[0] = (int)n0;
+        T.end[1] = (int)(n0 + n1);
+        T.end[2] = (int)(n0 + n1 + n2);
+        return T;
+    };
+    auto blocks = [&](int kind) { return batch_blocks(stage_box(kind, bx), kBlock, -1, 0, 0); };
+    auto grid = [](const Batch3 &T) { return dim3((unsigned)T.end[2]); };
+    Batch3 T = three(blocks(ST_G2), blocks(ST_DIVU), 0);
+    hipLaunchKernelGGL(k_flat_divu<false>, grid(T), dim3(kBlock), 0, st, T, hc.use_flattening,
+                       (int)CAMR_NGROW, (const DevFab *)nullptr, hc, (int *)nullptr);
+    T = three(face1_blocks(bx, 0), face1_blocks(bx, 1), face1_blocks(bx, 2));
+    if (hc.ppm_type == 1)
+        hipLaunchKernelGGL(k_face1_ppm, grid(T), dim3(kBlock), 0, st, T, hc, dtp);
+    else
+        hipLaunchKernelGGL(k_face1_plm, grid(T), dim3(kBlock), 0, st, T, has_src, hc, dtp);
+    T = three(blocks(ST_T1), blocks(ST_T1 + 1), blocks(ST_T1 + 2));
+    hipLaunchKernelGGL(k_trans1_all, grid(T), dim3(kBlock), 0, st, T, hc, dtp);
+    FluxOut o;
+    for (int d = 0; d < 3; ++d) o.f[d] = A.flx[d];
+    T = three(blocks(ST_T2), blocks(ST_T2 + 1), blocks(ST_T2 + 2));
+    if (has_src)
+        hipLaunchKernelGGL(k_trans2_box<1>, grid(T), dim3(kBlock), 0, st, T, hc, dtp, o);
+    else
+        hipLaunchKernelGGL(k_trans2_box<0>, grid(T), dim3(kBlock), 0, st, T, hc, dtp, o);
+    launch_one(k_box_update, ST_VALID, bx, B, st, A.dsdt, o, A.area_c[0], A.area_c[1], A.area_c[2],
                A.vol_c);
     return hipGetLastError() == hipSuccess ? CAMR_OK : CAMR_ERR_HIP;
 }

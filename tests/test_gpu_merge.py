@@ -1,0 +1,48 @@
+"""The transverse stages as one launch per direction and as one launch of
+all three (levels up to kMergeBlocks blocks): both against the oracle, bit
+for bit.  Block sizes that differ between the directions (or between the
+flattening and the nodal divergence) keep the launches apart at any size."""
+import numpy as np
+import pytest
+
+from camr_amd import workloads
+from camr_amd.hydro import Level, Problem
+from tests.test_gpu_parity import _oracle_params, assert_bitwise
+
+pytestmark = pytest.mark.gpu
+
+BOXES = [(0, 0, 0, 16, 11, 8), (17, 0, 0, 19, 11, 8)]  # 17 and 3 cells along x
+
+
+def _blocks(split):
+    b = [256] * 13
+    if split:
+        b[1], b[5], b[9] = 128, 64, 128  # flattening, x transdo, x final faces
+    return b
+
+
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("zm", [0, 2, 5])
+@pytest.mark.parametrize("grav", [0.0, -0.7])
+def test_merged_and_split_transverse_launches(oracle, split, zm, grav):
+    print(f"merge split={split} zm={zm} grav={grav}", flush=True)
+    prob = Problem(domlo=(0, 0, 0), domhi=(19, 11, 8), dx=(1 / 20,) * 3, bclo=(2, 0, 4),
+                   bchi=(4, 0, 2), is_periodic=(0, 1, 0), boxes=BOXES,
+                   params=dict(ppm_type=1, cfl=0.3, const_grav=grav))
+    o = oracle.Level(_oracle_params(oracle, prob), prob.boxes)
+    g = Level(prob)
+    g.tuning = (_blocks(split), 0)
+    z = g.zmarch
+    z[7] = z[11] = zm
+    g.zmarch = z
+    for b, bx in enumerate(BOXES):
+        U = workloads.smooth_field().state(20, bx[:3], bx[3:])
+        o.set_box(b, U)
+        g.set_box(b, U)
+    o.init_post()
+    g.init_post()
+    err, od = o.run(3)
+    assert err == 0
+    assert np.array_equal(od, g.run(3))
+    for b in range(len(BOXES)):
+        assert_bitwise(g.get_box(b), o.get_box(b), f"box {b}")
