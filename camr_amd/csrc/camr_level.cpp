@@ -1623,7 +1623,10 @@ int HydroLevel::advance(double dt) {
     std::swap(snew_, sold_);
     a_is_new_ = !a_is_new_;
     set_dt_dev(dt);
-    if (fused_ && !grav_src_values_) {
+    // with gravity, a coarse level of a hierarchy keeps the pass-by-pass
+    // sequence: its cleaned S_old is what the finer level's ghost cells are
+    // interpolated from in time
+    if (fused_ && !(grav_src_values_ && reg_crse_)) {
         rc = advance_fused(dt);
         pending_ = true;
         last_dt_ = dt;
@@ -1820,6 +1823,7 @@ int HydroLevel::advance_fused(double dt) {
     fa.dtp = dt_dev_;
     fa.g = desc_.const_grav;
     fa.add_grav = desc_.add_grav_src;
+    fa.src = grav_src_values_ ? engine_.grav_src() : SRC_NONE;
     PostArgs pa;
     pa.hc = hc_;
     pa.dtp = dt_dev_;
@@ -1831,8 +1835,8 @@ int HydroLevel::advance_fused(double dt) {
     for (int i = 0; i < nb; ++i) {
         const int b = batched_ ? -1 : i;
         int rc = engine_.fill(b, parity(), fa, stream_, status_, &prof_);
-        if (!rc) rc = engine_.hydro(b, parity(), true, nullptr, nullptr, 0, hc_, dt_dev_, stream_,
-                                    status_, &prof_, &pa);
+        if (!rc) rc = engine_.hydro(b, parity(), true, nullptr, nullptr, fa.src, hc_, dt_dev_,
+                                    stream_, status_, &prof_, &pa);
         if (rc) return rc;
     }
     dt_ready_ = true;
@@ -1910,6 +1914,7 @@ int HydroLevel::capture_graphs() {
         fa.dtp = dtp;
         fa.g = desc_.const_grav;
         fa.add_grav = desc_.add_grav_src;
+        fa.src = SRC_NONE;
         PostArgs pa;
         pa.hc = hc_;
         pa.dtp = dtp;
@@ -2189,6 +2194,7 @@ int HydroLevel::adjoint_step(double dt, bool check) {
     fa.dtp = dt_dev_;
     fa.g = desc_.const_grav;
     fa.add_grav = desc_.add_grav_src;
+    fa.src = SRC_NONE;
     rc = engine_.fill(-1, parity(), fa, stream_, status_, &prof_);
     // the update itself is applied in registers by the post-pass adjoint
     if (!rc) rc = engine_.hydro(-1, parity(), true, nullptr, nullptr, 0, hc_, dt_dev_, stream_,

@@ -42,6 +42,33 @@ __device__ __forceinline__ bool prim_compact(const double *v, double *o, double 
     return true;
 }
 
+// hydro_srctoprim (Hydro_ctoprim.H:106-157) of the conserved sources src of
+// a cell with state v and specific internal energy e, compact.
+__device__ __forceinline__ void src_compact(const double *v, double e, const double *src,
+                                            double *o) {
+    const double rho = v[URHO];
+    const double rhoinv = 1.0 / rho;
+    const double vx = v[UMX] * rhoinv, vy = v[UMY] * rhoinv, vz = v[UMZ] * rhoinv;
+    const double srcrho = src[URHO];
+    o[SR] = srcrho;
+    o[SU] = (src[UMX] - vx * srcrho) * rhoinv;
+    o[SV] = (src[UMY] - vy * srcrho) * rhoinv;
+    o[SW] = (src[UMZ] - vz * srcrho) * rhoinv;
+    const double sre = src[UEINT];
+    o[SE] = sre;
+#pragma unroll
+    for (int s = 0; s < NSPEC; ++s)
+        o[SY + s] = (src[UFS + s] - (v[UFS + s] * rhoinv) * srcrho) * rhoinv;
+    const double dpde = (kGamma - 1.0) * rho, dpdr = (kGamma - 1.0) * e;
+    o[SP] = dpde * (sre - (e * rho) * srcrho * rhoinv) * rhoinv + dpdr * srcrho;
+}
+
+// Primitive sources of a launch: none, all NS components in S_SRCQ, or a
+// constant gravity's, of which only the z velocity's is stored (the source
+// has no mass, momentum x / y, internal energy or species part, so that
+// hydro_srctoprim gives +0 for the others).
+enum { SRC_NONE = 0, SRC_ALL = 1, SRC_GRAV = 2 };
+
 // The same, stored at (i,j,k) of q.
 __device__ __forceinline__ void prim_compact_point(const double *v, const Arr &q, int i,
                                                    int j, int k, const HydroConst &hc,
@@ -366,6 +393,7 @@ struct FillArgs {
     const double *dtp;       // the step's dt (device)
     double g;
     int add_grav;
+    int src;  // SRC_*: what fill writes to S_SRCQ (SRC_ALL with zeros)
 };
 struct PostArgs {
     HydroConst hc;
@@ -429,8 +457,8 @@ class FusedEngine {
     // parity selects the table whose snew is buffer A (0) or B (1).
     // construct_hydro_source + the S_new Saxpy (snew += dt * dS/dt); floor
     // and energy checks into *status.  have_prim: fill() already wrote the
-    // primitives and the Sborder copy; else they come from sb_tab (and the
-    // primitive sources from src_tab when has_src).
+    // primitives, the Sborder copy and the primitive sources; else they come
+    // from sb_tab (and the sources from src_tab).  has_src: SRC_*.
     // With `post`, the update and the post pass (post()) run as one kernel;
     // with `no_update` the final update is left out (the fluxes are ready in
     // the scratch, S_new is not touched).
@@ -455,6 +483,8 @@ class FusedEngine {
     // adjoint arrays with the canonical layout of every box (allocated on
     // first use); total doubles of one scratch set
     int enable_adjoint();
+    // the gravity sources fill() writes: the CTU face kernels read them all
+    int grav_src() const { return tune_.ctu ? SRC_ALL : SRC_GRAV; }
     double *adjoint_base() const { return ascratch_.base(); }
     size_t scratch_total() const { return total_; }
 
@@ -481,6 +511,9 @@ class FusedEngine {
                  A... args);
     // block-prefix row rk (see kBlkRows), table entry range of box b
     LaunchCfg cfg_row(int rk, int b, int parity) const;
+    template <int SRC>
+    void trans2_launches(int b, int parity, const HydroConst &hc, const double *dtp,
+                         hipStream_t st, Prof *prof);
     bool merge_faces(int kind, int b, int parity, LaunchCfg c[3]) const;
     // grid of the trace + first-flux kernel of direction d
     LaunchCfg cfg_face1(int d, int b, int parity) const;

@@ -45,6 +45,17 @@ __device__ __forceinline__ unsigned shift(const Canon &L) {
 }
 
 
+// ------------------------------------------------------------ sources
+// Whether component s of the primitive sources is stored for a source kind
+// (SRC_*): the others are +0 everywhere.
+__device__ __forceinline__ constexpr bool has_comp(int src, int s) {
+    return src == SRC_ALL || (src == SRC_GRAV && s == SW);
+}
+template <int SRC>
+__device__ __forceinline__ double src_ld(const CView &sq, unsigned v, int s) {
+    return has_comp(SRC, s) ? sq.ld(v, s) : 0.0;
+}
+
 // ------------------------------------------------------------ primitives
 // hydro_ctoprim (Hydro_ctoprim.H:11-101) into the compact layout, with
 // hydro_srctoprim (:106-157) when sources are non-zero; also copies Sborder
@@ -89,20 +100,12 @@ k_prim_c(Batch B, const DevFab *sb_tab, const DevFab *src_tab, int has_src, Hydr
     for (int n = 0; n < NQC; ++n) q.st(v0, n, o[n]);
     if (has_src) {
         const CView sq = cview(L, srcq_, NS);
-        const double rhoinv = 1.0 / rho;
-        const double vx = v[UMX] * rhoinv, vy = v[UMY] * rhoinv, vz = v[UMZ] * rhoinv;
-        const double srcrho = src(i, j, k, URHO);
-        sq.st(v0, SR, srcrho);
-        sq.st(v0, SU, (src(i, j, k, UMX) - vx * srcrho) * rhoinv);
-        sq.st(v0, SV, (src(i, j, k, UMY) - vy * srcrho) * rhoinv);
-        sq.st(v0, SW, (src(i, j, k, UMZ) - vz * srcrho) * rhoinv);
-        const double sre = src(i, j, k, UEINT);
-        sq.st(v0, SE, sre);
+        double sv[NVAR], o9[NS];
 #pragma unroll
-        for (int s = 0; s < NSPEC; ++s)
-            sq.st(v0, SY + s, (src(i, j, k, UFS + s) - (v[UFS + s] * rhoinv) * srcrho) * rhoinv);
-        const double dpde = (kGamma - 1.0) * rho, dpdr = (kGamma - 1.0) * e;
-        sq.st(v0, SP, dpde * (sre - (e * rho) * srcrho * rhoinv) * rhoinv + dpdr * srcrho);
+        for (int n = 0; n < NVAR; ++n) sv[n] = src(i, j, k, n);
+        src_compact(v, e, sv, o9);
+#pragma unroll
+        for (int n = 0; n < NS; ++n) sq.st(v0, n, o9[n]);
     }
 }
 
@@ -255,7 +258,7 @@ __device__ __forceinline__ void plm_cell(const CView &q, const CView &sq, int ha
 #pragma unroll
             for (int o = -2; o <= 2; ++o) {
                 rr[o + 2] = q.ld(v0 + (unsigned)o * sd, SR);
-                gg[o + 2] = has_src ? sq.ld(v0 + (unsigned)o * sd, SU + D) : 0.0;
+                gg[o + 2] = has_comp(has_src, SU + D) ? sq.ld(v0 + (unsigned)o * sd, SU + D) : 0.0;
             }
             sl[s] = mc_pslope(st, rr, gg, hc.dx[D], fl, hc.plm_iorder);
         } else {
@@ -538,7 +541,7 @@ __device__ __forceinline__ void trans2_point(const Batch &B, int w, int nw, cons
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             n[s] = qp.ld(v0, s);
-            src[s] = HAS_SRC ? sq.ld(v0, s) : 0.0;
+            src[s] = src_ld<HAS_SRC>(sq, v0, s);
         }
         TransDiff t;
         trans2_diff<D>(v0, L, Fa, Fb, ca, cb, t);
@@ -550,7 +553,7 @@ __device__ __forceinline__ void trans2_point(const Batch &B, int w, int nw, cons
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             n[s] = qm.ld(v0, s);
-            src[s] = HAS_SRC ? sq.ld(vm, s) : 0.0;
+            src[s] = src_ld<HAS_SRC>(sq, vm, s);
         }
         TransDiff t;
         trans2_diff<D>(vm, L, Fa, Fb, ca, cb, t);
@@ -705,7 +708,7 @@ k_trans2_zm(Batch B, HydroConst hc, const double *dtp) {
     unsigned v = L.off(i, j, k0 - 1);
     trans2_diff<2>(v, L, Fa, Fb, ca, cb, tm);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) srcm[s] = HAS_SRC ? sq.ld(v, s) : 0.0;
+    for (int s = 0; s < NS; ++s) srcm[s] = src_ld<HAS_SRC>(sq, v, s);
 #pragma unroll
     for (int n = 0; n < NVAR; ++n) um[n] = uc.ld(v, n);
     double cm = q.ld(v, SC), csm = q.ld(v, SCS);
@@ -719,7 +722,7 @@ k_trans2_zm(Batch B, HydroConst hc, const double *dtp) {
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
                 n[s] = qp.ld(v, s);
-                srcp[s] = HAS_SRC ? sq.ld(v, s) : 0.0;
+                srcp[s] = src_ld<HAS_SRC>(sq, v, s);
             }
             transverse_two_d(n, tp, hdt, srcp, hc.trd, hc.small_pres, sp);
         }
@@ -888,12 +891,12 @@ __device__ __forceinline__ void trans2_x_point(const Batch &B, int w, int nw,
         double n[NS], srcp[NS], srcm[NS];
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            srcp[s] = HAS_SRC ? sq.ld(v0, s) : 0.0;
-            srcm[s] = HAS_SRC ? lane_up(srcp[s]) : 0.0;
+            srcp[s] = src_ld<HAS_SRC>(sq, v0, s);
+            srcm[s] = has_comp(HAS_SRC, s) ? lane_up(srcp[s]) : 0.0;
         }
         if (HAS_SRC && own) {
 #pragma unroll
-            for (int s = 0; s < NS; ++s) srcm[s] = sq.ld(vm, s);
+            for (int s = 0; s < NS; ++s) srcm[s] = src_ld<HAS_SRC>(sq, vm, s);
         }
         TransDiff tp, tm;
         trans2_diff<0>(v0, L, Fa, Fb, ca, cb, tp);
@@ -1122,7 +1125,7 @@ __device__ __forceinline__ void ctu_face(const BoxEnt &E, const Canon &L, unsign
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             n[s] = qp.ld(v, s);
-            src[s] = HAS_SRC ? sq.ld(v, s) : 0.0;
+            src[s] = src_ld<HAS_SRC>(sq, v, s);
         }
         transverse_two_d(n, tp, hdt, src, hc.trd, hc.small_pres, sp);
     }
@@ -1131,7 +1134,7 @@ __device__ __forceinline__ void ctu_face(const BoxEnt &E, const Canon &L, unsign
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             n[s] = qm.ld(v, s);
-            src[s] = HAS_SRC ? sq.ld(v - sd, s) : 0.0;
+            src[s] = src_ld<HAS_SRC>(sq, v - sd, s);
         }
         transverse_two_d(n, tm, hdt, src, hc.trd, hc.small_pres, sm);
     }
@@ -1840,11 +1843,27 @@ void FusedEngine::launch_ctu(const char *name, Prof *prof, K kern, int d, int b,
     hipLaunchKernelGGL(kern, dim3(c.grid), dim3(kCtuBlock), 0, st, c.B, args...);
 }
 
+template <int SRC>
+void FusedEngine::trans2_launches(int b, int parity, const HydroConst &hc, const double *dtp,
+                                  hipStream_t st, Prof *prof) {
+    LaunchCfg c[3];
+    if (merge_faces(ST_T2, b, parity, c)) {
+        launch3("transverse_2", prof, k_trans2_all<SRC>, c, st, hc, dtp);
+        return;
+    }
+    launch("transverse_2", prof, k_trans2<0, SRC>, ST_T2 + 0, b, parity, st, hc, dtp);
+    launch("transverse_2", prof, k_trans2<1, SRC>, ST_T2 + 1, b, parity, st, hc, dtp);
+    if (tune_.zm[ST_T2 + 2] > 0)
+        launch("transverse_2", prof, k_trans2_zm<SRC>, ST_T2 + 2, b, parity, st, hc, dtp);
+    else
+        launch("transverse_2", prof, k_trans2<2, SRC>, ST_T2 + 2, b, parity, st, hc, dtp);
+}
+
 int FusedEngine::hydro(int b, int parity, bool have_prim, const DevFab *sb_tab,
                        const DevFab *src_tab, int has_src, const HydroConst &hc,
                        const double *dtp, hipStream_t st, int *status, Prof *prof,
                        const PostArgs *post, bool no_update) {
-    if (!have_prim || has_src)
+    if (!have_prim)
         launch("prim", prof, k_prim_c, ST_G4, b, parity, st, sb_tab, src_tab, has_src, hc, status);
     // q beyond the canonical grow(bx, 4) comes from sb_tab (given with !have_prim)
     const int qgrow = (!have_prim && sb_tab) ? qgrow_ : CAMR_NGROW;
@@ -1894,25 +1913,9 @@ int FusedEngine::hydro(int b, int parity, bool have_prim, const DevFab *sb_tab,
             else
                 launch("transverse_1", prof, k_trans1<2>, ST_T1 + 2, b, parity, st, hc, dtp);
         }
-        const bool zm2 = tune_.zm[ST_T2 + 2] > 0;
-        if (merge_faces(ST_T2, b, parity, c)) {
-            if (has_src) launch3("transverse_2", prof, k_trans2_all<1>, c, st, hc, dtp);
-            else launch3("transverse_2", prof, k_trans2_all<0>, c, st, hc, dtp);
-        } else if (has_src) {
-            launch("transverse_2", prof, k_trans2<0, 1>, ST_T2 + 0, b, parity, st, hc, dtp);
-            launch("transverse_2", prof, k_trans2<1, 1>, ST_T2 + 1, b, parity, st, hc, dtp);
-            if (zm2)
-                launch("transverse_2", prof, k_trans2_zm<1>, ST_T2 + 2, b, parity, st, hc, dtp);
-            else
-                launch("transverse_2", prof, k_trans2<2, 1>, ST_T2 + 2, b, parity, st, hc, dtp);
-        } else {
-            launch("transverse_2", prof, k_trans2<0, 0>, ST_T2 + 0, b, parity, st, hc, dtp);
-            launch("transverse_2", prof, k_trans2<1, 0>, ST_T2 + 1, b, parity, st, hc, dtp);
-            if (zm2)
-                launch("transverse_2", prof, k_trans2_zm<0>, ST_T2 + 2, b, parity, st, hc, dtp);
-            else
-                launch("transverse_2", prof, k_trans2<2, 0>, ST_T2 + 2, b, parity, st, hc, dtp);
-        }
+        if (has_src == SRC_GRAV) trans2_launches<SRC_GRAV>(b, parity, hc, dtp, st, prof);
+        else if (has_src) trans2_launches<SRC_ALL>(b, parity, hc, dtp, st, prof);
+        else trans2_launches<SRC_NONE>(b, parity, hc, dtp, st, prof);
     }
     if (no_update) {
         // the caller applies the update itself
@@ -2025,9 +2028,9 @@ int fused_umdrv(const UmdrvArgs &A, double dt, double *scratch, hipStream_t st) 
     for (int d = 0; d < 3; ++d) o.f[d] = A.flx[d];
     T = three(blocks(ST_T2), blocks(ST_T2 + 1), blocks(ST_T2 + 2));
     if (has_src)
-        hipLaunchKernelGGL(k_trans2_box<1>, grid(T), dim3(kBlock), 0, st, T, hc, dtp, o);
+        hipLaunchKernelGGL(k_trans2_box<SRC_ALL>, grid(T), dim3(kBlock), 0, st, T, hc, dtp, o);
     else
-        hipLaunchKernelGGL(k_trans2_box<0>, grid(T), dim3(kBlock), 0, st, T, hc, dtp, o);
+        hipLaunchKernelGGL(k_trans2_box<SRC_NONE>, grid(T), dim3(kBlock), 0, st, T, hc, dtp, o);
     launch_one(k_box_update, ST_VALID, bx, B, st, A.dsdt, o, A.area_c[0], A.area_c[1], A.area_c[2],
                A.vol_c);
     return hipGetLastError() == hipSuccess ? CAMR_OK : CAMR_ERR_HIP;
