@@ -186,6 +186,7 @@ class HydroLevel {
     int clean_state(std::vector<Arr> &S, bool launch_detect);
     int expand_state();
     int construct_hydro_source(double dt, bool add = true);
+    int read_back();
     int check_status();
     int status_error(int st);
     void release();
@@ -201,6 +202,8 @@ class HydroLevel {
     std::vector<Arr> snew_, sold_, sbv_;
     DevFab *tab_old_ = nullptr, *tab_sb_ = nullptr, *tab_src_ = nullptr;
     int *owner_ = nullptr;
+    // device: one allocation {dtmin_, status_}, mirrored by one pinned host
+    // block, so that a step's end is read back by a single copy
     int *status_ = nullptr;              // device: error bits | floor flag
     int *redo_ = nullptr;                // device: the staged tail must be repeated pass by pass
     unsigned long long *dtmin_ = nullptr;  // device: bit pattern of min dt
@@ -292,6 +295,7 @@ class HydroLevel {
     bool pending_ = false;   // a fused step awaits resolve()
     bool needs_ext_ = false; // some ghost cell has no owning box
     bool dt_ready_ = false;  // dtmin_ holds the CFL estimate of S_new
+    bool dt_host_ = false;   // and *h_dtmin_ is a copy of it
     double last_dt_ = 0.0;
     DevFab *tab_a_ = nullptr, *tab_b_ = nullptr;  // raw-state tables of buffers A / B
     DevFab *tab_dsdt_ = nullptr;                  // staged engine: dS/dt of every box
@@ -687,7 +691,7 @@ void HydroLevel::release() {
     exp_box_.clear();
     fr(tab_old_); fr(tab_sb_); fr(tab_src_); fr(tab_a_); fr(tab_b_); fr(tab_dsdt_);
     tab_dsdt_ = nullptr;
-    tab_a_ = tab_b_ = nullptr; fr(owner_); fr(status_); fr(redo_); fr(dtmin_);
+    tab_a_ = tab_b_ = nullptr; fr(owner_); fr(redo_); fr(dtmin_);
     redo_ = nullptr;
     fr(dt_dev_); fr(ext_); dt_dev_ = nullptr; ext_ = nullptr;
     release_graphs();
@@ -720,7 +724,6 @@ void HydroLevel::release() {
     nws_ = 0;
     for (auto p : ebbuf_) fr(p);
     ebbuf_.clear();
-    if (h_status_) (void)hipHostFree(h_status_);
     if (h_dtmin_) (void)hipHostFree(h_dtmin_);
     tab_old_ = tab_sb_ = tab_src_ = nullptr;
     owner_ = status_ = nullptr;
@@ -880,14 +883,14 @@ int HydroLevel::create() {
         for (int b = 0; b < nb; ++b) t[b].a = dense(srchyd_[b], grow(box_[b], CAMR_NGROW));
         CAMR_HIP(hipMemcpy(tab_src_, t.data(), nb * sizeof(DevFab), hipMemcpyHostToDevice));
     }
-    CAMR_HIP(hipMalloc(&status_, sizeof(int)));
     CAMR_HIP(hipMalloc(&redo_, sizeof(int)));
     CAMR_HIP(hipMemset(redo_, 0, sizeof(int)));
-    CAMR_HIP(hipMalloc(&dtmin_, sizeof(unsigned long long)));
+    CAMR_HIP(hipMalloc(&dtmin_, 2 * sizeof(unsigned long long)));
+    status_ = (int *)(dtmin_ + 1);
     CAMR_HIP(hipMalloc(&dt_dev_, sizeof(double)));
     CAMR_HIP(hipMemset(status_, 0, sizeof(int)));
-    CAMR_HIP(hipHostMalloc(&h_status_, sizeof(int)));
-    CAMR_HIP(hipHostMalloc(&h_dtmin_, sizeof(unsigned long long)));
+    CAMR_HIP(hipHostMalloc(&h_dtmin_, 2 * sizeof(unsigned long long)));
+    h_status_ = (int *)(h_dtmin_ + 1);
     // the fused engine implements the Godunov integrator only
     fused_ = (desc_.engine != 1) && !desc_.hp.do_mol;
     batched_ = desc_.batched != 0;
@@ -1407,10 +1410,17 @@ int HydroLevel::state_array(int b, camr_array4 *out) {
     return CAMR_OK;
 }
 
-int HydroLevel::check_status() {
-    CAMR_HIP(hipMemcpyAsync(h_status_, status_, sizeof(int), hipMemcpyDeviceToHost, stream_));
+// Waits for the level's stream and reads dtmin_ and status_ back.
+int HydroLevel::read_back() {
+    CAMR_HIP(hipMemcpyAsync(h_dtmin_, dtmin_, 2 * sizeof(unsigned long long),
+                            hipMemcpyDeviceToHost, stream_));
     CAMR_HIP(hipStreamSynchronize(stream_));
-    return status_error(*h_status_);
+    return CAMR_OK;
+}
+
+int HydroLevel::check_status() {
+    const int rc = read_back();
+    return rc ? rc : status_error(*h_status_);
 }
 
 // The error of the device status word `st` (already read back): the first
@@ -1436,10 +1446,8 @@ int HydroLevel::status_error(int st) {
 }
 
 int HydroLevel::sync() {
-    int rc = resolve();
-    if (rc) return rc;
-    CAMR_HIP(hipStreamSynchronize(stream_));
-    return check_status();
+    const int rc = resolve();
+    return rc ? rc : check_status();
 }
 
 int HydroLevel::init_post() {
@@ -1622,11 +1630,13 @@ int HydroLevel::advance(double dt) {
     // swapTimeLevels (CAMR_advance.cpp:72-75)
     std::swap(snew_, sold_);
     a_is_new_ = !a_is_new_;
-    set_dt_dev(dt);
+    dt_host_ = false;
     // with gravity, a coarse level of a hierarchy keeps the pass-by-pass
     // sequence: its cleaned S_old is what the finer level's ghost cells are
     // interpolated from in time
-    if (fused_ && !(grav_src_values_ && reg_crse_)) {
+    const bool fused = fused_ && !(grav_src_values_ && reg_crse_);
+    if (!fused) set_dt_dev(dt);
+    if (fused) {
         rc = advance_fused(dt);
         pending_ = true;
         last_dt_ = dt;
@@ -1810,9 +1820,8 @@ int HydroLevel::hydro_on_workers(double dt) {
 // density floor fires, which resolve() detects and answers with
 // advance_exact from the untouched raw S_old.
 int HydroLevel::advance_fused(double dt) {
-    (void)dt;
-    const unsigned long long init = (unsigned long long)0x7fefffffffffffffULL;  // DBL_MAX
-    launch_on(k_fill_u64, make_box1(), stream_, dtmin_, init);
+    hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(64), 0, stream_, dt_dev_, dt, dtmin_,
+                       (unsigned long long)0x7fefffffffffffffULL /* DBL_MAX */);
     FillArgs fa;
     fa.sold_tab = a_is_new_ ? tab_b_ : tab_a_;  // table of the buffers now old
     fa.owner = owner_;
@@ -1981,6 +1990,7 @@ int HydroLevel::run_graph(int nsteps, double *dts) {
         int rc = capture_graphs();
         if (rc) return rc;
     }
+    dt_host_ = false;
     int done = 0;
     double dt_old = 0.0;
     bool first = true;
@@ -2564,8 +2574,9 @@ int HydroLevel::adj_download(int b, double *h) {
 int HydroLevel::resolve() {
     if (!pending_) return CAMR_OK;
     pending_ = false;
-    CAMR_HIP(hipMemcpyAsync(h_status_, status_, sizeof(int), hipMemcpyDeviceToHost, stream_));
-    CAMR_HIP(hipStreamSynchronize(stream_));
+    int rb = read_back();
+    if (rb) return rb;
+    dt_host_ = dt_ready_;
     if (*h_status_ & kFloorFlag) {
         *h_status_ &= ~kFloorFlag;
         CAMR_HIP(hipMemcpyAsync(status_, h_status_, sizeof(int), hipMemcpyHostToDevice, stream_));
@@ -2583,7 +2594,7 @@ int HydroLevel::resolve() {
             CAMR_HIP(hipStreamSynchronize(stream_));
         }
     }
-    return check_status();
+    return status_error(*h_status_);
 }
 
 // estTimeStep (CAMR.cpp:490-563)
@@ -2601,10 +2612,13 @@ int HydroLevel::est_time_step(double *est) {
                    hc_.dx[1], hc_.dx[2], dtmin_, status_, ebf_);
         CAMR_HIP(hipGetLastError());
         dt_ready_ = true;
+        dt_host_ = false;
     }
-    CAMR_HIP(hipMemcpyAsync(h_dtmin_, dtmin_, sizeof(unsigned long long), hipMemcpyDeviceToHost, stream_));
-    int rc = sync();
-    if (rc) return rc;
+    if (!dt_host_) {
+        const int rc = check_status();
+        if (rc) return rc;
+        dt_host_ = true;
+    }
     double dt;
     unsigned long long bits = *h_dtmin_;
     memcpy(&dt, &bits, sizeof(dt));
@@ -3331,6 +3345,87 @@ void camr_default_level_desc(camr_level_desc *d) {
 const char *camr_last_error(void) { return g_err; }
 int camr_version(void) { return 100; }
 
+} // extern "C"
+
+namespace {
+// A few words of device memory and their pinned host mirror, for the
+// synchronous per-box calls that return a device result.  Taken for one
+// call (so calls of several threads and streams never share them) and put
+// back after it; up to kKeep sets per device are kept for later calls, more
+// are freed.  Bytes 0..31 hold anything, the status word at byte 32 is zero
+// in a kept set.
+class CallWords {
+  public:
+    static constexpr size_t kBytes = 64, kStatus = 32;
+    CallWords() {
+        if (hipGetDevice(&dev_) != hipSuccess) return;
+        if (dev_ < kDevices) {
+            std::lock_guard<std::mutex> g(mu());
+            Kept &k = kept(dev_);
+            if (k.n > 0) {
+                s_ = k.s[--k.n];
+                return;
+            }
+        }
+        if (hipMalloc(&s_.dev, kBytes) != hipSuccess) { s_.dev = nullptr; return; }
+        if (hipHostMalloc(&s_.host, kBytes) != hipSuccess || !zero_status()) drop();
+    }
+    // after the call's work has ended: the words may be kept, their status
+    // word being `status`
+    void finished(int status) { keep_ = status == 0 || zero_status(); }
+    ~CallWords() {
+        if (!s_.dev) return;
+        if (keep_ && dev_ < kDevices) {
+            std::lock_guard<std::mutex> g(mu());
+            Kept &k = kept(dev_);
+            if (k.n < kKeep) {
+                k.s[k.n++] = s_;
+                return;
+            }
+        }
+        drop();  // hipFree waits for what an early return left running
+    }
+    CallWords(const CallWords &) = delete;
+    CallWords &operator=(const CallWords &) = delete;
+    bool ok() const { return s_.dev != nullptr; }
+    char *dev() const { return (char *)s_.dev; }
+    char *host() const { return (char *)s_.host; }
+    int *status() const { return (int *)(dev() + kStatus); }
+
+  private:
+    struct Set {
+        void *dev, *host;
+    };
+    static constexpr int kKeep = 16, kDevices = 16;
+    struct Kept {
+        int n;
+        Set s[kKeep];
+    };
+    static std::mutex &mu() {
+        static std::mutex m;
+        return m;
+    }
+    static Kept &kept(int dev) {
+        static Kept k[kDevices];  // zero-initialised
+        return k[dev];
+    }
+    bool zero_status() {
+        return hipMemset(s_.dev, 0, kBytes) == hipSuccess &&
+               hipStreamSynchronize(nullptr) == hipSuccess;
+    }
+    void drop() {
+        if (s_.dev) (void)hipFree(s_.dev);
+        if (s_.host) (void)hipHostFree(s_.host);
+        s_ = Set{nullptr, nullptr};
+    }
+    int dev_ = 0;
+    bool keep_ = false;
+    Set s_{nullptr, nullptr};
+};
+} // namespace
+
+extern "C" {
+
 int camr_hydro_ctoprim(const camr_box *qbx, const camr_array4 *u, const camr_array4 *q,
                        const camr_array4 *qaux, const camr_hydro_params *p, void *stream) {
     if (!qbx || !u || !q || !qaux || !p) { set_error("null argument"); return CAMR_ERR_PARAM; }
@@ -3340,14 +3435,13 @@ int camr_hydro_ctoprim(const camr_box *qbx, const camr_array4 *u, const camr_arr
         return CAMR_ERR_SHAPE;
     }
     hipStream_t s = (hipStream_t)stream;
-    int *st = nullptr;
-    CAMR_HIP(hipMallocAsync(&st, sizeof(int), s));
-    CAMR_HIP(hipMemsetAsync(st, 0, sizeof(int), s));
-    launch_on(k_ctoprim, B, s, view(*u), view(*q), view(*qaux), make_const(*p), st);
-    int h = 0;
-    CAMR_HIP(hipMemcpyAsync(&h, st, sizeof(int), hipMemcpyDeviceToHost, s));
-    CAMR_HIP(hipFreeAsync(st, s));
+    CallWords w;
+    if (!w.ok()) { set_error("camr_hydro_ctoprim: status word"); return CAMR_ERR_ALLOC; }
+    launch_on(k_ctoprim, B, s, view(*u), view(*q), view(*qaux), make_const(*p), w.status());
+    CAMR_HIP(hipMemcpyAsync(w.host(), w.status(), sizeof(int), hipMemcpyDeviceToHost, s));
     CAMR_HIP(hipStreamSynchronize(s));
+    const int h = *(const int *)w.host();
+    w.finished(h);
     if (h & (1 << CAMR_ERR_NEG_ENERGY)) {
         set_error("rho E or rho e not positive (Hydro_ctoprim.H:56,68)");
         return CAMR_ERR_NEG_ENERGY;
@@ -3625,15 +3719,18 @@ int camr_estdt_hydro(const camr_box *bx, const camr_array4 *u, const double dx[3
     const Box B = make_box(bx->lo, bx->hi);
     if (!covers(*u, B, NVAR)) { set_error("u must cover bx"); return CAMR_ERR_SHAPE; }
     hipStream_t s = (hipStream_t)stream;
-    struct { unsigned long long m; int st; int pad; } h = {0x7fefffffffffffffULL, 0, 0};
-    char *buf = nullptr;
-    CAMR_HIP(hipMallocAsync((void **)&buf, 16, s));
-    CAMR_HIP(hipMemcpyAsync(buf, &h, 16, hipMemcpyHostToDevice, s));
+    struct Result { unsigned long long m; int st; int pad; } h = {0x7fefffffffffffffULL, 0, 0};
+    CallWords w;
+    if (!w.ok()) { set_error("camr_estdt_hydro: result words"); return CAMR_ERR_ALLOC; }
+    char *buf = w.dev();
+    *(Result *)w.host() = h;
+    CAMR_HIP(hipMemcpyAsync(buf, w.host(), 16, hipMemcpyHostToDevice, s));
     launch_on(k_estdt, B, s, view(*u), dx[0], dx[1], dx[2], (unsigned long long *)buf, (int *)(buf + 8),
               EbFlags{});
-    CAMR_HIP(hipMemcpyAsync(&h, buf, 16, hipMemcpyDeviceToHost, s));
-    CAMR_HIP(hipFreeAsync(buf, s));
+    CAMR_HIP(hipMemcpyAsync(w.host(), buf, 16, hipMemcpyDeviceToHost, s));
     CAMR_HIP(hipStreamSynchronize(s));
+    h = *(const Result *)w.host();
+    w.finished(0);
     if (h.st & (1 << CAMR_ERR_DT)) { set_error("ERROR: dt needs to be positive."); return CAMR_ERR_DT; }
     double v;
     memcpy(&v, &h.m, sizeof(v));

@@ -337,6 +337,16 @@ __global__ void k_fill_u64(Range r, unsigned long long *p, unsigned long long v)
     if (blockIdx.x == 0 && threadIdx.x == 0) *p = v;
 }
 
+// The two words a fused step starts from: its dt and the minimum its CFL
+// estimate is reduced into.
+__global__ void k_step_begin(double *dtp, double dt, unsigned long long *dtmin,
+                             unsigned long long v) {
+    if (threadIdx.x == 0) {
+        *dtp = dt;
+        *dtmin = v;
+    }
+}
+
 // ----------------------------------------------------- device dt control
 // First node of a captured level step: estTimeStep + computeNewDt (or
 // computeInitialDt on the first step) of CAMR.cpp:474-676 from the CFL
