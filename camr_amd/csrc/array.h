@@ -92,6 +92,7 @@ __host__ __device__ inline Range range_of(const Box &b) {
 // dimension: entry u owns blocks [off[u], off[u + 1]).  n = 0: a 2-D grid,
 // blockIdx.y the entry and blockIdx.x its block (for longer tables).
 constexpr int kFlatEntries = 64;
+constexpr int kGridRows = 65535;  // grid.y: entries of one launch when not flattened
 struct FlatBlocks {
     int n;
     int off[kFlatEntries + 1];

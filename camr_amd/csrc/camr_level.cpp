@@ -259,6 +259,10 @@ class HydroLevel {
     // boxes).  tab_sbx_ / tab_dsdtx_: the level's rows, then one per
     // virtual box
     bool eb_merge_ = true;
+    // the cut-cell boxes' / the adjoint's scratch has a buffer per transverse
+    // pair (EbBox::keep)
+    bool eb_keep_ = false, eadj_keep_ = false;
+    bool eb_keep(const std::vector<Box> &bs) const;
     std::vector<Box> vbox_;
     int nmerged_ = 0;
     int *vg_ids_ = nullptr;
@@ -1017,6 +1021,10 @@ int HydroLevel::set_eb(const int32_t *flags, const int32_t flo[3], const int32_t
     cut_cells_h_.clear();
     size_t tot = 0;
     auto r32 = [](size_t n) { return (n + 31) / 32 * 32; };
+    std::vector<Box> cut;
+    for (int b = 0; b < nb; ++b)
+        if (kind_[b] == 1) cut.push_back(box_[b]);
+    eb_keep_ = eb_keep(cut);
     for (int b = 0; b < nb; ++b) {
         if (kind_[b] != 1) continue;
         const Box B = box_[b], G = grow(B, ng_);
@@ -1024,7 +1032,7 @@ int HydroLevel::set_eb(const int32_t *flags, const int32_t flo[3], const int32_t
         cut_off_.push_back(tot);
         tot += r32((size_t)(2 * QVAR + NQAUX) * G.npts());
         for (int d = 0; d < 3; ++d) tot += r32((size_t)NVAR * nodes(B, d).npts());
-        tot += r32(umdrv_eb_scratch_doubles(B, G));
+        tot += r32(umdrv_eb_scratch_doubles(B, G, eb_keep_));
     }
     if (!cut_ids_.empty()) {
         CAMR_HIP(hipMalloc(&cut_buf_, tot * sizeof(double)));
@@ -1343,6 +1351,20 @@ int HydroLevel::set_box_eb(int b, const double *vf, const double *const ap[3],
     return rc;
 }
 
+// Whether boxes bs run all transverse pairs in one launch (EbBox::keep): not
+// where the memory that takes beyond pair by pair (0.4 of the boxes' scratch)
+// is more than an eighth of what is free, so that a large level and what is
+// allocated after it still fit.
+bool HydroLevel::eb_keep(const std::vector<Box> &bs) const {
+    size_t more = 0, free_b = 0, total_b = 0;
+    for (const Box &B : bs) {
+        const Box G = grow(B, ng_);
+        more += umdrv_eb_scratch_doubles(B, G, true) - umdrv_eb_scratch_doubles(B, G, false);
+    }
+    return eb_merge_ && hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
+           more * sizeof(double) <= free_b / 8;
+}
+
 // Table entry c of the cut-cell batch: box cut_ids_[c] with its arrays in
 // cut_buf_ (q, qaux, srcq over grow(bx, 6), the face fluxes, the scratch),
 // its Sborder, dS/dt and geometry; copied to the device table.
@@ -1369,7 +1391,7 @@ int HydroLevel::cut_entry(int c) {
     }
     A.has_src = 0;
     A.g = ebg_[b];
-    eb_box_setup(A, p, &cut_htab_[c]);
+    eb_box_setup(A, p, &cut_htab_[c], eb_keep_);
     CAMR_HIP(hipMemcpy(cut_tab_ + c, &cut_htab_[c], sizeof(EbBox), hipMemcpyHostToDevice));
     return CAMR_OK;
 }
@@ -2292,13 +2314,16 @@ int HydroLevel::eb_adjoint_setup() {
         for (size_t v = 0; v < vbox_.size(); ++v) eadj_ids_.push_back(-1 - (int)v);
         auto r32 = [](size_t n) { return (n + 31) / 32 * 32; };
         size_t fn = 0, an = 0;
+        std::vector<Box> run;
+        for (int id : eadj_ids_) run.push_back(id >= 0 ? box_[id] : vbox_[-1 - id]);
+        eadj_keep_ = eb_keep(run);
         for (int id : eadj_ids_) {
             const Box B = id >= 0 ? box_[id] : vbox_[-1 - id], G = grow(B, ng_);
             fn += r32((size_t)(QVAR + NQAUX) * G.npts());
             for (int d = 0; d < 3; ++d) fn += r32((size_t)NVAR * nodes(B, d).npts());
             fn += r32(umdrv_eb_scratch_doubles(B, G, true));
             an += r32((size_t)(QVAR + NQAUX) * G.npts());
-            an += r32(umdrv_eb_scratch_doubles(B, G, false));
+            an += r32(umdrv_eb_scratch_doubles(B, G, eadj_keep_));
         }
         for (int b = 0; b < nb; ++b)
             an += r32((size_t)NVAR * box_[b].npts()) + r32((size_t)NVAR * grow(box_[b], ng_).npts());
@@ -2394,14 +2419,14 @@ int HydroLevel::eb_adjoint_setup() {
         ap += r32((size_t)(QVAR + NQAUX) * G.npts());
         Ab.uin = id >= 0 ? sbbv[id] : vga[v].sb;
         Ab.dsdt = id >= 0 ? ubv[id] : vub[v];
-        // the adjoint side shares one buffer of face states among the pairs
-        // and one among the final solves (set, not accumulated)
-        eb_box_setup(Ab, ap, &eadj_h_[c].A, false);
-        ap += r32(umdrv_eb_scratch_doubles(B, G, false));
+        // the adjoints of the pairs' and final solves' face states are set,
+        // not accumulated: they need no clearing
+        eb_box_setup(Ab, ap, &eadj_h_[c].A, eadj_keep_);
+        ap += r32(umdrv_eb_scratch_doubles(B, G, eadj_keep_));
         eadj_h_[c].F = eadj_fh_[c];
         const EbBox &Ad = eadj_h_[c].A;
         const size_t x0 = (size_t)(Ad.qmT[0].p - eadj_abuf_);
-        const size_t x1 = (size_t)(Ad.qpF[0].p - eadj_abuf_) +
+        const size_t x1 = (size_t)(Ad.qpF[2].p - eadj_abuf_) +
                           (size_t)NS * layout_of(B, G).bxg1.npts();
         skip.push_back({x0, x1});
     }
@@ -3703,11 +3728,18 @@ int camr_hydro_umdrv_eb(const camr_box *bx, const camr_array4 *uin, const camr_a
     for (int d = 0; d < 3; ++d) { A.g.ap[d] = view(geom->ap[d]); A.g.fc[d] = view(geom->fc[d]); }
     hipStream_t s = (hipStream_t)stream;
     double *scr = nullptr;
-    const size_t n = umdrv_eb_scratch_doubles(B, A.qbox);
-    CAMR_HIP(hipMallocAsync((void **)&scr, (n + 1) * sizeof(double), s));
+    // (where the larger scratch is not to be had: pair by pair)
+    bool keep = true;
+    size_t n = umdrv_eb_scratch_doubles(B, A.qbox, keep);
+    if (hipMallocAsync((void **)&scr, (n + 1) * sizeof(double), s) != hipSuccess) {
+        (void)hipGetLastError();
+        keep = false;
+        n = umdrv_eb_scratch_doubles(B, A.qbox, keep);
+        CAMR_HIP(hipMallocAsync((void **)&scr, (n + 1) * sizeof(double), s));
+    }
     A.dtp = scr + n;
     put_double(scr + n, dt, s);
-    rc = umdrv_eb(A, scr, s);
+    rc = umdrv_eb(A, scr, keep, s);
     CAMR_HIP(hipFreeAsync(scr, s));
     if (rc) { set_error("kernel launch failed"); return rc; }
     return CAMR_OK;

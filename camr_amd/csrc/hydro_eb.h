@@ -129,33 +129,35 @@ struct EbBox {
     Arr QM[3], QP[3], F1[3], G1[3], F2[3][3], G2[3][3], FT[3], QE[3];
     // the corrected states of transverse pair p (D|T in the order 0|1, 0|2,
     // 1|0, 1|2, 2|0, 2|1) and the final states of direction d: one buffer
-    // for all pairs / all directions, or one each when the adjoint reads
-    // them back (`keep`)
+    // each (`keep`), so that all pairs run in one launch and all directions
+    // in another, or one for all, which then go one after the other
     Arr qmT[6], qpT[6], qmF[3], qpF[3];
+    bool keep() const { return qmT[1].p != qmT[0].p; }
     Arr divu, divc, wt, optmp0, delm, winv;
     int regular;  // UmdrvEbArgs::regular
     int noflx;    // 1: the face fluxes of bx are not copied into flx (a recompute)
 };
 
 // Doubles of scratch one box needs (the one-box call's EbBox record
-// included); keep: every pair's and direction's states in their own arrays.
-size_t umdrv_eb_scratch_doubles(const Box &bx, const Box &qbox, bool keep = false);
+// included); keep: every pair's and direction's states in their own arrays
+// (126 more doubles per cell, about 0.4 of the rest).
+size_t umdrv_eb_scratch_doubles(const Box &bx, const Box &qbox, bool keep);
 // Carves the scratch arrays of box A.bx out of `scratch` (device memory of
 // umdrv_eb_scratch_doubles(A.bx, A.qbox, keep) doubles) into *out (host
 // memory).
-void eb_box_setup(const UmdrvEbArgs &A, double *scratch, EbBox *out, bool keep = false);
+void eb_box_setup(const UmdrvEbArgs &A, double *scratch, EbBox *out, bool keep);
 // hydro_umdrv_eb over the n boxes of tab (device copy) / htab (the same
-// records in host memory, read for the grid sizes): one launch per stage,
-// every box of the table in the launch.  All boxes share hc, dtp and has_src
-// (srcq holds primitive sources).
+// records in host memory, read for the grid sizes; all of one `keep`): one
+// launch per group of independent stages, every box in the launch.  All
+// boxes share hc, dtp and has_src (srcq holds primitive sources).
 // A cut cell (eb_type kEbSingle) of grow(bx, 2) of entry e of a table.
 struct CutCell {
     int e, i, j, k;
 };
 // cells (device, ncells): every cut cell of grow(bx, 2) of the table's
 // boxes; the cut-cell divergence and the redistribution's source side then
-// run over them alone (one thread per cut cell) instead of over grow(bx, 2)
-// and grow(bx, 1).
+// run over them alone (one thread per component of a cut cell) instead of
+// over grow(bx, 2) and grow(bx, 1).
 int umdrv_eb_batch(const EbBox *tab, const EbBox *htab, int n, const HydroConst &hc,
                    const double *dtp, int has_src, hipStream_t st, Prof *prof = nullptr,
                    const CutCell *cells = nullptr, int ncells = 0);
@@ -165,7 +167,8 @@ int eb_prim_batch(const EbBox *tab, const EbBox *htab, int n, const HydroConst &
                   hipStream_t st, Prof *prof = nullptr);
 // One box: its EbBox record goes into the head of scratch (written by a
 // kernel, so the call can be captured into a graph).
-int umdrv_eb(const UmdrvEbArgs &A, double *scratch, hipStream_t st, Prof *prof = nullptr);
+int umdrv_eb(const UmdrvEbArgs &A, double *scratch, bool keep, hipStream_t st,
+             Prof *prof = nullptr);
 // Per valid cell of bx: the wall momentum flux of its cut cell times dx2
 // (3 components, 0 for other cells) into out; q / qaux cover bx.
 int eb_force_box(const Box &bx, Arr q, Arr qaux, const EbGeom &g, const HydroConst &hc, Arr out,

@@ -324,7 +324,9 @@ template <bool CUT>
 CAMR_HD void
 b_eb_div(int i, int j, int k, Box bx, Arr ft0, Arr ft1, Arr ft2, Arr ge0, Arr ge1, Arr ge2, EbGeom g,
          Arr q, Arr qaux, Arr divc, Arr wt, Arr fo0, Arr fo1, Arr fo2, HydroConst hc,
-         double dxi0, double dxi1, double dxi2, bool out = true) {
+         double dxi0, double dxi1, double dxi2, bool out = true, int n0 = 0, int n1 = NVAR) {
+    // n0, n1: the components [n0, n1) of a cut cell (the list kernel's
+    // threads take one each; a cell's components do not depend on each other)
     const int32_t w = g.f(i, j, k);
     if (eb_type(w) == kEbCovered) return;
     // CUT: the cut cells only; otherwise the regular cells and the weight of
@@ -365,7 +367,7 @@ b_eb_div(int i, int j, int k, Box bx, Arr ft0, Arr ft1, Arr ft2, Arr ge0, Arr ge
         double fw[NVAR];
         eb_wallflux(q, qaux, g, i, j, k, hc, fw);
 #pragma unroll 1
-        for (int n = 0; n < NVAR; ++n) {
+        for (int n = n0; n < n1; ++n) {
             const double fxm = centroid_value<0>(ft0, n, g, i, j, k);
             const double fxp = centroid_value<0>(ft0, n, g, i + 1, j, k);
             const double fym = centroid_value<1>(ft1, n, g, i, j, k);
@@ -381,9 +383,14 @@ b_eb_div(int i, int j, int k, Box bx, Arr ft0, Arr ft1, Arr ft2, Arr ge0, Arr ge
                 if (zh) fo2(i, j, k + 1, n) = fzp;
             }
             double dvv = cvi / vfr * (axp * fxp - axm * fxm + ayp * fyp - aym * fym + azp * fzp - azm * fzm);
-            dvv += fw[n] * dxi0 / vfr;
+            double fwn = 0.0;  // fw[n] without indexing registers by n
+#pragma unroll
+            for (int m = 0; m < NVAR; ++m) fwn = m == n ? fw[m] : fwn;
+            dvv += fwn * dxi0 / vfr;
             divc(i, j, k, n) = dvv * -1.0;
         }
+        if (n0 == 0) wt(i, j, k, 0) = q(i, j, k, QRHO);
+        if (UEINT < n0 || UEINT >= n1) return;
         const double fxm = axm > 0.0 ? centroid_value<0>(ge0, GUN, g, i, j, k) : 0.0;
         const double fxp = axp > 0.0 ? centroid_value<0>(ge0, GUN, g, i + 1, j, k) : 0.0;
         const double fym = aym > 0.0 ? centroid_value<1>(ge1, GUN, g, i, j, k) : 0.0;
@@ -393,7 +400,6 @@ b_eb_div(int i, int j, int k, Box bx, Arr ft0, Arr ft1, Arr ft2, Arr ge0, Arr ge
         divc(i, j, k, UEINT) -= (1.0 / vfr) * q(i, j, k, QPRES) *
                                 (dxi0 * (axp * fxp - axm * fxm) + dxi1 * (ayp * fyp - aym * fym) +
                                  dxi2 * (azp * fzp - azm * fzm));
-        wt(i, j, k, 0) = q(i, j, k, QRHO);
     }
 }
 
@@ -402,13 +408,14 @@ b_eb_div(int i, int j, int k, Box bx, Arr ft0, Arr ft1, Arr ft2, Arr ge0, Arr ge
 // registers, use_wts_in_divnc false), over grow(bx, 1): the cut cell's
 // own share optmp0 and the mass deficit delm it hands out, and 1 / (sum of
 // its neighbours' weight * vfrac).
+// [n0, n1): the components done here; with n0 = 0 also 1 / (...).
 CAMR_HD void
-b_redist_src(int i, int j, int k, EbGeom g, Box dbox2, Arr divc, Arr wt, Arr optmp0, Arr delm, Arr winv) {
+b_redist_src(int i, int j, int k, EbGeom g, Box dbox2, Arr divc, Arr wt, Arr optmp0, Arr delm, Arr winv,
+             int n0 = 0, int n1 = NVAR) {
     const int32_t w = g.f(i, j, k);
     if (eb_type(w) != kEbSingle) {
-#pragma unroll
-        for (int n = 0; n < NVAR; ++n) { optmp0(i, j, k, n) = 0.0; delm(i, j, k, n) = 0.0; }
-        winv(i, j, k, 0) = 0.0;
+        for (int n = n0; n < n1; ++n) { optmp0(i, j, k, n) = 0.0; delm(i, j, k, n) = 0.0; }
+        if (n0 == 0) winv(i, j, k, 0) = 0.0;
         return;
     }
     const double vfc = g.vf(i, j, k, 0);
@@ -427,7 +434,7 @@ b_redist_src(int i, int j, int k, EbGeom g, Box dbox2, Arr divc, Arr wt, Arr opt
         vtot += g.vf(i + t % 3 - 1, j + (t / 3) % 3 - 1, k + t / 9 - 1, 0) * 1.0;
     }
 #pragma unroll 1
-    for (int n = 0; n < NVAR; ++n) {
+    for (int n = n0; n < n1; ++n) {
         double divnc = 0.0;
         for (uint32_t m = in; m; m &= m - 1) {
             const int t = __builtin_ctz(m);
@@ -440,6 +447,7 @@ b_redist_src(int i, int j, int k, EbGeom g, Box dbox2, Arr divc, Arr wt, Arr opt
         optmp0(i, j, k, n) = op;
         delm(i, j, k, n) = -(vfc) * op;
     }
+    if (n0 != 0) return;
     double wtot = 0.0;
     for (uint32_t m = con; m; m &= m - 1) {
         const int t = __builtin_ctz(m);
@@ -475,18 +483,25 @@ b_redist_dst(int i, int j, int k, EbGeom g, Box dbox2, Arr divc, Arr wt, Arr opt
     // the cell's own share (zero unless it is a cut cell; b_redist_src
     // writes that zero when it runs over every cell, not over a cell list)
     const bool own = eb_type(g.f(i, j, k)) == kEbSingle;
-#pragma unroll 1
-    for (int n = 0; n < NVAR; ++n) {
-        double acc = own ? optmp0(i, j, k, n) : 0.0;
-        // in increasing bit order: k, then j, then i of the sender
-        for (uint32_t m = src; m; m &= m - 1) {
-            const int t = __builtin_ctz(m);
-            const int ok = t / 9 - 1, oj = (t / 3) % 3 - 1, oi = t % 3 - 1;
-            const double drho = delm(i + oi, j + oj, k + ok, n) * winv(i + oi, j + oj, k + ok, 0) * wtt * mask;
-            acc += drho;
+    // (sender by sender, so that a sender's ten loads are in flight at once:
+    // component by component the cells beside a cut held the launch up for
+    // 64 us at 2 boxes of 32^3)
+    double acc[NVAR];
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) acc[n] = own ? optmp0(i, j, k, n) : 0.0;
+    // in increasing bit order: k, then j, then i of the sender
+    for (uint32_t m = src; m; m &= m - 1) {
+        const int t = __builtin_ctz(m);
+        const int ok = t / 9 - 1, oj = (t / 3) % 3 - 1, oi = t % 3 - 1;
+        const double wi = winv(i + oi, j + oj, k + ok, 0);
+#pragma unroll
+        for (int n = 0; n < NVAR; ++n) {
+            const double drho = delm(i + oi, j + oj, k + ok, n) * wi * wtt * mask;
+            acc[n] += drho;
         }
-        dsdt(i, j, k, n) = divc(i, j, k, n) + acc;
     }
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) dsdt(i, j, k, n) = divc(i, j, k, n) + acc[n];
 }
 
 CAMR_HD void
@@ -495,9 +510,8 @@ b_zero(int i, int j, int k, Arr a, int nc) {
 }
 
 // ---------------------------------------------------------------- driver
-// The stages of hydro_umdrv_eb in launch order: one launch site each, run
-// over every box of a table (grid.y = box).  The transverse pairs D|T go in
-// the order of Godunov_3D_eb.cpp:214-455, (0|1, 0|2, 1|0, 1|2, 2|0, 2|1),
+// The stages of hydro_umdrv_eb in order, each run over every box of a
+// table.  The transverse pairs D|T go in the order of Godunov_3D_eb.cpp:214-455, (0|1, 0|2, 1|0, 1|2, 2|0, 2|1),
 // each as transdo then Riemann; the final states per direction as transdd
 // then Riemann.
 enum EbSite {
@@ -601,12 +615,10 @@ CAMR_HD void site_body(const EbBox &B, const Layout &L, int i, int j, int k,
     }
 }
 
+// Block lb of site S on box B.
 template <int S>
-__global__ void __launch_bounds__(kBlock)
-k_eb_site(const EbBox *tab, HydroConst hc, const double *dtp, int has_src, FlatBlocks fb) {
-    int u, lb;
-    flat_entry(fb, u, lb);
-    const EbBox &B = tab[u];
+__device__ __forceinline__ void site_block(const EbBox &B, int lb, const HydroConst &hc,
+                                           const double *dtp, int has_src) {
     if constexpr (S == ES_DIVCUT || S == ES_RSRC)
         if (B.regular) return;
     const Layout L = layout_of(B.bx, B.qbox);
@@ -629,20 +641,26 @@ constexpr const char *site_name(int s) {
          : s <= ES_DIVCUT ? "eb_divergence" : "eb_redistribute";
 }
 
-// The cut-cell divergence over a list of the cut cells.
+// The cut-cell divergence over a list of the cut cells, one component per
+// block row (grid.y = NVAR).  A few thousand cells are a handful of blocks,
+// so the time is one thread's chain of dependent loads: all ten components
+// in a thread took 110 us at 1.2e3 cells.
 __global__ void __launch_bounds__(kBlock)
-k_eb_divcut_list(const EbBox *tab, const CutCell *cells, int n, HydroConst hc, const double *dtp,
-                 int has_src) {
+k_eb_divcut_list(const EbBox *tab, const CutCell *cells, int n, HydroConst hc) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
     const CutCell c = cells[t];
     const EbBox &B = tab[c.e];
-    const Layout L = layout_of(B.bx, B.qbox);
-    site_body<ES_DIVCUT>(B, L, c.i, c.j, c.k, hc, dtp, has_src);
+    if (B.regular) return;  // no cut cell
+    const int m = (int)blockIdx.y;
+    b_eb_div<true>(c.i, c.j, c.k, B.bx, B.FT[0], B.FT[1], B.FT[2], B.QE[0], B.QE[1], B.QE[2], B.g,
+                   B.q, B.qaux, B.divc, B.wt, B.flx[0], B.flx[1], B.flx[2], hc, 1.0 / hc.dx[0],
+                   1.0 / hc.dx[1], 1.0 / hc.dx[2], !B.noflx, m, m + 1);
 }
 
 // The redistribution's source side over the cut cells of grow(bx, 1) in
-// the list (the other cells send nothing).
+// the list (the other cells send nothing), one component per block row
+// (123 us with all ten in a thread).
 __global__ void __launch_bounds__(kBlock)
 k_eb_rsrc_list(const EbBox *tab, const CutCell *cells, int n) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -650,42 +668,109 @@ k_eb_rsrc_list(const EbBox *tab, const CutCell *cells, int n) {
     const CutCell c = cells[t];
     const EbBox &B = tab[c.e];
     if (!grow(B.bx, 1).contains(c.i, c.j, c.k)) return;
-    b_redist_src(c.i, c.j, c.k, B.g, B.dbox2, B.divc, B.wt, B.optmp0, B.delm, B.winv);
+    const int m = (int)blockIdx.y;
+    b_redist_src(c.i, c.j, c.k, B.g, B.dbox2, B.divc, B.wt, B.optmp0, B.delm, B.winv, m, m + 1);
 }
 
+// Blocks of site S over the n boxes of htab, none where the stage has no
+// point or nothing to do there.
 template <int S>
-void launch_site(const EbBox *tab, const EbBox *htab, int n, const HydroConst &hc,
-                 const double *dtp, int has_src, hipStream_t st, Prof *prof,
-                 const CutCell *cells, int ncells) {
-    if ((S == ES_DIVCUT || S == ES_RSRC) && cells) {
-        if (ncells == 0) return;
-        Region reg(prof, site_name(S), st);
-        if (S == ES_DIVCUT)
-            hipLaunchKernelGGL(k_eb_divcut_list, dim3(grid_for(ncells)), dim3(kBlock), 0, st, tab,
-                               cells, ncells, hc, dtp, has_src);
-        else
-            hipLaunchKernelGGL(k_eb_rsrc_list, dim3(grid_for(ncells)), dim3(kBlock), 0, st, tab,
-                               cells, ncells);
-        return;
-    }
-    // blocks per box: none where the stage has no point or nothing to do
-    auto cnt = [&](int b) -> int64_t {
-        if ((S == ES_DIVCUT || S == ES_RSRC) && htab[b].regular) return 0;
-        const Box sb = site_box<S>(htab[b], layout_of(htab[b].bx, htab[b].qbox));
-        return sb.ok() ? (sb.npts() + kBlock - 1) / kBlock : 0;
-    };
-    FlatBlocks fb;
-    const dim3 grid = flat_blocks(n, cnt, fb);
-    if (grid.x == 0) return;
-    Region reg(prof, site_name(S), st);
-    hipLaunchKernelGGL(k_eb_site<S>, grid, dim3(kBlock), 0, st, tab, hc, dtp, has_src, fb);
+int64_t site_blocks(const EbBox &B) {
+    if ((S == ES_DIVCUT || S == ES_RSRC) && B.regular) return 0;
+    const Box sb = site_box<S>(B, layout_of(B.bx, B.qbox));
+    return sb.ok() ? (sb.npts() + kBlock - 1) / kBlock : 0;
 }
 
+// One launch of sites that do not read each other's results, over every box
+// of the table: entry u of the launch is site s0 + u / n of the list on box
+// u % n.
 template <int... S>
-void launch_sites(std::integer_sequence<int, S...>, const EbBox *tab, const EbBox *htab, int n,
-                  const HydroConst &hc, const double *dtp, int has_src, hipStream_t st,
-                  Prof *prof, const CutCell *cells, int ncells) {
-    (launch_site<S>(tab, htab, n, hc, dtp, has_src, st, prof, cells, ncells), ...);
+__global__ void __launch_bounds__(kBlock)
+k_eb_sites(const EbBox *tab, int n, int s0, HydroConst hc, const double *dtp, int has_src,
+           FlatBlocks fb) {
+    int u, lb;
+    flat_entry(fb, u, lb);
+    const int si = u / n;
+    const EbBox &B = tab[u - si * n];
+    int q = -s0;
+    ((q++ == si ? site_block<S>(B, lb, hc, dtp, has_src) : (void)0), ...);
+}
+
+// The sites [s0, s1) of the list, kGridRows entries to a launch (grid.y, where
+// the entries are too many to be flattened).
+template <int... S>
+void launch_group(const EbBox *tab, const EbBox *htab, int n, const HydroConst &hc,
+                  const double *dtp, int has_src, hipStream_t st, Prof *prof, int s0 = 0,
+                  int s1 = (int)sizeof...(S)) {
+    typedef int64_t (*Count)(const EbBox &);
+    const Count counts[] = {site_blocks<S>...};
+    constexpr int sites[] = {S...};
+    const int per = kGridRows / (s1 - s0);
+    for (int b0 = 0; b0 < n; b0 += per) {
+        const int m = std::min(per, n - b0);
+        FlatBlocks fb;
+        const dim3 grid = flat_blocks(
+            (s1 - s0) * m, [&](int u) { return counts[s0 + u / m](htab[b0 + u % m]); }, fb);
+        if (grid.x == 0) continue;
+        Region reg(prof, site_name(sites[s0]), st);
+        hipLaunchKernelGGL((k_eb_sites<S...>), grid, dim3(kBlock), 0, st, tab + b0, m, s0, hc, dtp,
+                           has_src, fb);
+    }
+}
+
+// hydro_umdrv_eb's stages in order, stages that are independent of each
+// other in one launch: 11 launches where one per stage took 32.  Boxes whose
+// pairs share a buffer (EbBox::keep) go pair by pair.
+void launch_all_sites(const EbBox *tab, const EbBox *htab, int n, const HydroConst &hc,
+                      const double *dtp, int has_src, hipStream_t st, Prof *prof,
+                      const CutCell *cells, int ncells) {
+#define CAMR_EB_GO(...) launch_group<__VA_ARGS__>(tab, htab, n, hc, dtp, has_src, st, prof)
+    auto pair_states = [&](int s0, int s1) {
+        launch_group<ES_PAIR + 0, ES_PAIR + 2, ES_PAIR + 4, ES_PAIR + 6, ES_PAIR + 8, ES_PAIR + 10,
+                     ES_DIVU>(tab, htab, n, hc, dtp, has_src, st, prof, s0, s1);
+    };
+    auto pair_solves = [&](int s0, int s1) {
+        launch_group<ES_PAIR + 1, ES_PAIR + 3, ES_PAIR + 5, ES_PAIR + 7, ES_PAIR + 9, ES_PAIR + 11>(
+            tab, htab, n, hc, dtp, has_src, st, prof, s0, s1);
+    };
+    auto final_states = [&](int s0, int s1) {
+        launch_group<ES_FINAL + 0, ES_FINAL + 2, ES_FINAL + 4>(tab, htab, n, hc, dtp, has_src, st,
+                                                               prof, s0, s1);
+    };
+    auto final_solves = [&](int s0, int s1) {
+        launch_group<ES_FINAL + 1, ES_FINAL + 3, ES_FINAL + 5>(tab, htab, n, hc, dtp, has_src, st,
+                                                               prof, s0, s1);
+    };
+    // (the zero fill rides with a stage of few registers: with the trace's
+    // 185 it took 396 us for the two, apart 300)
+    CAMR_EB_GO(ES_PLM);
+    CAMR_EB_GO(ES_R1 + 0, ES_R1 + 1, ES_R1 + 2, ES_ZERO);
+    if (htab[0].keep()) {
+        pair_states(0, 7);
+        pair_solves(0, 6);
+        final_states(0, 3);
+        final_solves(0, 3);
+    } else {
+        pair_states(6, 7);
+        for (int p = 0; p < 6; ++p) { pair_states(p, p + 1); pair_solves(p, p + 1); }
+        for (int d = 0; d < 3; ++d) { final_states(d, d + 1); final_solves(d, d + 1); }
+    }
+    CAMR_EB_GO(ES_ADJ + 0, ES_ADJ + 1, ES_ADJ + 2);
+    CAMR_EB_GO(ES_DIV);
+    if (!cells) {
+        CAMR_EB_GO(ES_DIVCUT);
+        CAMR_EB_GO(ES_RSRC);
+    } else if (ncells > 0) {
+        const dim3 g(grid_for(ncells), NVAR);
+        {
+            Region reg(prof, site_name(ES_DIVCUT), st);
+            hipLaunchKernelGGL(k_eb_divcut_list, g, dim3(kBlock), 0, st, tab, cells, ncells, hc);
+        }
+        Region reg(prof, site_name(ES_RSRC), st);
+        hipLaunchKernelGGL(k_eb_rsrc_list, g, dim3(kBlock), 0, st, tab, cells, ncells);
+    }
+    CAMR_EB_GO(ES_RDST);
+#undef CAMR_EB_GO
 }
 
 // The EbBox of a one-box call, written into device memory by kernel
@@ -828,14 +913,13 @@ int umdrv_eb_batch(const EbBox *tab, const EbBox *htab, int n, const HydroConst 
                    const double *dtp, int has_src, hipStream_t st, Prof *prof,
                    const CutCell *cells, int ncells) {
     if (n <= 0) return CAMR_OK;
-    launch_sites(std::make_integer_sequence<int, ES_COUNT>{}, tab, htab, n, hc, dtp, has_src, st,
-                 prof, cells, ncells);
+    launch_all_sites(tab, htab, n, hc, dtp, has_src, st, prof, cells, ncells);
     return hipGetLastError() == hipSuccess ? CAMR_OK : CAMR_ERR_HIP;
 }
 
-int umdrv_eb(const UmdrvEbArgs &A, double *scratch, hipStream_t st, Prof *prof) {
+int umdrv_eb(const UmdrvEbArgs &A, double *scratch, bool keep, hipStream_t st, Prof *prof) {
     EbBox hb;
-    eb_box_setup(A, scratch + kEbHead, &hb);
+    eb_box_setup(A, scratch + kEbHead, &hb, keep);
     static_assert(sizeof(EbBox) % 8 == 0, "EbBox words");
     const int nw = (int)(sizeof(EbBox) / 8);
     const uint64_t *src = reinterpret_cast<const uint64_t *>(&hb);

@@ -199,27 +199,37 @@ CAMR_HD void adj_rdst(const EbBox &F, const EbBox &A, int i, int j, int k,
                 if (eb_type(ws) == kEbSingle && eb_conn(ws, -oi, -oj, -ok))
                     src |= 1u << ((oi + 1) + 3 * (oj + 1) + 9 * (ok + 1));
             }
-    double wttb = 0.0;
+    double db[NH], wttb = 0.0;
+#pragma unroll
     for (int n = 0; n < NH; ++n) {
-        const double db = dt * A.dsdt(i, j, k, n);
-        if (db == 0.0) continue;
-        A.divc(i, j, k, n) += db;
-        A.optmp0(i, j, k, n) += db;
-        for (uint32_t m = src; m; m &= m - 1) {
-            const int t = __builtin_ctz(m);
-            const int ok = t / 9 - 1, oj = (t / 3) % 3 - 1, oi = t % 3 - 1;
+        db[n] = dt * A.dsdt(i, j, k, n);
+        if (db[n] == 0.0) continue;
+        A.divc(i, j, k, n) += db[n];
+        A.optmp0(i, j, k, n) += db[n];
+    }
+    // sender by sender (b_redist_dst)
+    for (uint32_t m = src; m; m &= m - 1) {
+        const int t = __builtin_ctz(m);
+        const int ok = t / 9 - 1, oj = (t / 3) % 3 - 1, oi = t % 3 - 1;
+        const double wi = F.winv(i + oi, j + oj, k + ok, 0);
+        double wib = 0.0;
+#pragma unroll
+        for (int n = 0; n < NH; ++n) {
+            if (db[n] == 0.0) continue;
             const double dl = F.delm(i + oi, j + oj, k + ok, n);
-            const double wi = F.winv(i + oi, j + oj, k + ok, 0);
-            aadd(A.delm, i + oi, j + oj, k + ok, n, db * wi * wtt * mask);
-            aadd(A.winv, i + oi, j + oj, k + ok, 0, db * dl * wtt * mask);
-            wttb += db * dl * wi * mask;
+            aadd(A.delm, i + oi, j + oj, k + ok, n, db[n] * wi * wtt * mask);
+            wib += db[n] * dl * wtt * mask;
+            wttb += db[n] * dl * wi * mask;
         }
+        aadd(A.winv, i + oi, j + oj, k + ok, 0, wib);
     }
     aadd(A.wt, i, j, k, 0, wttb);
 }
 
 // b_redist_src in reverse (single cells only; the others wrote zeros).
-CAMR_HD void adj_rsrc(const EbBox &F, const EbBox &A, int i, int j, int k) {
+// part: -1 the whole cell, else component part of it (part 0 also the sum
+// of the weights); the list kernel's threads take a part each.
+CAMR_HD void adj_rsrc(const EbBox &F, const EbBox &A, int i, int j, int k, int part = -1) {
     if (F.regular) return;
     const EbGeom &g = F.g;
     const int32_t w = g.f(i, j, k);
@@ -238,7 +248,7 @@ CAMR_HD void adj_rsrc(const EbBox &F, const EbBox &A, int i, int j, int k) {
         const int t = __builtin_ctz(m);
         vtot += g.vf(i + t % 3 - 1, j + (t / 3) % 3 - 1, k + t / 9 - 1, 0) * 1.0;
     }
-    for (int n = 0; n < NH; ++n) {
+    for (int n = part < 0 ? 0 : part; n < (part < 0 ? NH : part + 1); ++n) {
         const double opb = A.optmp0(i, j, k, n) + A.delm(i, j, k, n) * -(vfc);
         if (opb == 0.0) continue;
         const double xb = opb * (1 - vfc) * mask;  // of divnc - divc(i)
@@ -251,7 +261,7 @@ CAMR_HD void adj_rsrc(const EbBox &F, const EbBox &A, int i, int j, int k) {
             aadd(A.divc, i + ii, j + jj, k + kk, n, sb * wf);
         }
     }
-    const double wib = A.winv(i, j, k, 0);
+    const double wib = part <= 0 ? A.winv(i, j, k, 0) : 0.0;
     if (wib != 0.0) {
         double wtot = 0.0;
         for (uint32_t m = con; m; m &= m - 1) {
@@ -273,9 +283,11 @@ CAMR_HD void adj_rsrc(const EbBox &F, const EbBox &A, int i, int j, int k) {
 
 // ------------------------------------------------------- hydro_consup_eb
 // b_eb_div in reverse.  CUT: the cut cells; otherwise the regular ones.
+// part: -1 the whole cell; of a cut cell 0..NH-1 the face fluxes of that
+// component, NH the wall flux and the weight, NH + 1 the p div u term.
 template <bool CUT>
 CAMR_HD void adj_div(const EbBox &F, const EbBox &A, int i, int j, int k,
-                                        const HydroConst &hc) {
+                                        const HydroConst &hc, int part = -1) {
     const EbGeom &g = F.g;
     const int32_t w = g.f(i, j, k);
     if (eb_type(w) == kEbCovered) return;
@@ -283,7 +295,7 @@ CAMR_HD void adj_div(const EbBox &F, const EbBox &A, int i, int j, int k,
     const double dxi0 = 1.0 / hc.dx[0], dxi1 = 1.0 / hc.dx[1], dxi2 = 1.0 / hc.dx[2];
     const double cvi = dxi0 * dxi1 * dxi2;
     // wt = rho
-    aadd(A.q, i, j, k, QRHO, A.wt(i, j, k, 0));
+    if (part < 0 || part == NH) aadd(A.q, i, j, k, QRHO, A.wt(i, j, k, 0));
     if constexpr (!CUT) {
         for (int n = 0; n < NH; ++n) {
             const double vb = -A.divc(i, j, k, n);
@@ -318,11 +330,10 @@ CAMR_HD void adj_div(const EbBox &F, const EbBox &A, int i, int j, int k,
         const double aym = g.ap[1](i, j, k, 0), ayp = g.ap[1](i, j + 1, k, 0);
         const double azm = g.ap[2](i, j, k, 0), azp = g.ap[2](i, j, k + 1, 0);
         const double vfr = g.vf(i, j, k, 0);
-        double fwb[NVAR] = {};
         for (int n = 0; n < NH; ++n) {
+            if (part >= 0 && part != n) continue;
             const double vb = -A.divc(i, j, k, n);
             if (vb == 0.0) continue;
-            fwb[n] = vb * dxi0 / vfr;
             const double sb = vb * (cvi / vfr);
             centroid_adj<0>(A.FT[0], n, g, i, j, k, -sb * axm);
             centroid_adj<0>(A.FT[0], n, g, i + 1, j, k, sb * axp);
@@ -332,7 +343,13 @@ CAMR_HD void adj_div(const EbBox &F, const EbBox &A, int i, int j, int k,
             centroid_adj<2>(A.FT[2], n, g, i, j, k + 1, sb * azp);
         }
         // wall flux of the cell
-        {
+        if (part < 0 || part == NH) {
+            double fwb[NVAR] = {};
+#pragma unroll
+            for (int n = 0; n < NH; ++n) {
+                const double vb = -A.divc(i, j, k, n);
+                if (vb != 0.0) fwb[n] = vb * dxi0 / vfr;
+            }
             const double wv[6] = {F.q(i, j, k, QRHO), F.q(i, j, k, QU), F.q(i, j, k, QV),
                                   F.q(i, j, k, QW), F.q(i, j, k, QPRES), F.q(i, j, k, QREINT)};
             double wb[6] = {};
@@ -345,7 +362,7 @@ CAMR_HD void adj_div(const EbBox &F, const EbBox &A, int i, int j, int k,
             aadd(A.qaux, i, j, k, QCSML, csb);
         }
         // eb_pdivu: divc(UEINT) -= (1 / vfr) p (sum_d dxi_d (a+ u+ - a- u-))
-        const double Pb = -A.divc(i, j, k, UEINT);
+        const double Pb = part < 0 || part == NH + 1 ? -A.divc(i, j, k, UEINT) : 0.0;
         if (Pb != 0.0) {
             const double fxm = axm > 0.0 ? centroid_value<0>(F.QE[0], GUN, g, i, j, k) : 0.0;
             const double fxp = axp > 0.0 ? centroid_value<0>(F.QE[0], GUN, g, i + 1, j, k) : 0.0;
@@ -882,12 +899,10 @@ CAMR_HD void adj_body(const EbBox &F, const EbBox &A, int i, int j, int k,
     else adj_prim(F, A, i, j, k, hc);
 }
 
+// Block lb of adjoint stage S on entry E.
 template <int S>
-__global__ void __launch_bounds__(kBlock)
-k_eb_adj_site(const EbAdjEnt *tab, HydroConst hc, const double *dtp, FlatBlocks fb) {
-    int u, lb;
-    flat_entry(fb, u, lb);
-    const EbAdjEnt &E = tab[u];
+__device__ __forceinline__ void adj_block(const EbAdjEnt &E, int lb, const HydroConst &hc,
+                                          const double *dtp) {
     if constexpr (S == AS_DIVCUT || S == AS_RSRC)
         if (E.F.regular) return;
     const Layout L = layout_of(E.F.bx, E.F.qbox);
@@ -910,49 +925,121 @@ constexpr const char *adj_name(int s) {
          : s == AS_PLM ? "ebadj_trace_plm" : "ebadj_ctoprim";
 }
 
-// AS_DIVCUT / AS_RSRC over a list of the cut cells
+// AS_DIVCUT / AS_RSRC over a list of the cut cells, one part of a cell per
+// block row: the list is a few blocks, so a thread's chain of loads and
+// atomics is the time (105 and 167 us with whole cells).
 template <int S>
 __global__ void __launch_bounds__(kBlock)
-k_eb_adj_list(const EbAdjEnt *tab, const CutCell *cells, int n, HydroConst hc,
-              const double *dtp) {
+k_eb_adj_list(const EbAdjEnt *tab, const CutCell *cells, int n, HydroConst hc) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
     const CutCell c = cells[t];
     const EbAdjEnt &E = tab[c.e];
-    if (S == AS_RSRC && !grow(E.F.bx, 1).contains(c.i, c.j, c.k)) return;
-    adj_body<S>(E.F, E.A, c.i, c.j, c.k, hc, *dtp);
+    const int part = (int)blockIdx.y;
+    if constexpr (S == AS_RSRC) {
+        if (!grow(E.F.bx, 1).contains(c.i, c.j, c.k)) return;
+        adj_rsrc(E.F, E.A, c.i, c.j, c.k, part);
+    } else {
+        if (!E.F.regular) adj_div<true>(E.F, E.A, c.i, c.j, c.k, hc, part);
+    }
 }
 
 template <int S>
-void launch_adj(const EbAdjEnt *tab, const EbAdjEnt *htab, int n, const HydroConst &hc,
-                const double *dtp, hipStream_t st, Prof *prof, const CutCell *cells,
-                int ncells) {
-    if constexpr (S == AS_DIVCUT || S == AS_RSRC) {
-        if (cells) {
-            if (ncells == 0) return;
-            Region reg(prof, adj_name(S), st);
-            hipLaunchKernelGGL(k_eb_adj_list<S>, dim3(grid_for(ncells)), dim3(kBlock), 0, st,
-                               tab, cells, ncells, hc, dtp);
-            return;
-        }
-    }
-    auto cnt = [&](int b) -> int64_t {
-        if ((S == AS_DIVCUT || S == AS_RSRC) && htab[b].F.regular) return 0;
-        const Box sb = adj_box<S>(htab[b].F, layout_of(htab[b].F.bx, htab[b].F.qbox));
-        return sb.ok() ? (sb.npts() + kBlock - 1) / kBlock : 0;
-    };
-    FlatBlocks fb;
-    const dim3 grid = flat_blocks(n, cnt, fb);
-    if (grid.x == 0) return;
-    Region reg(prof, adj_name(S), st);
-    hipLaunchKernelGGL(k_eb_adj_site<S>, grid, dim3(kBlock), 0, st, tab, hc, dtp, fb);
+int64_t adj_blocks(const EbAdjEnt &E) {
+    if ((S == AS_DIVCUT || S == AS_RSRC) && E.F.regular) return 0;
+    const Box sb = adj_box<S>(E.F, layout_of(E.F.bx, E.F.qbox));
+    return sb.ok() ? (sb.npts() + kBlock - 1) / kBlock : 0;
 }
 
+// One launch of adjoint stages that do not read each other's results: entry
+// u is stage s0 + u / n of the list on box u % n.
 template <int... S>
-void launch_adjs(std::integer_sequence<int, S...>, const EbAdjEnt *tab, const EbAdjEnt *htab,
-                 int n, const HydroConst &hc, const double *dtp, hipStream_t st, Prof *prof,
-                 const CutCell *cells, int ncells) {
-    (launch_adj<S>(tab, htab, n, hc, dtp, st, prof, cells, ncells), ...);
+__global__ void __launch_bounds__(kBlock)
+k_eb_adj_sites(const EbAdjEnt *tab, int n, int s0, HydroConst hc, const double *dtp,
+               FlatBlocks fb) {
+    int u, lb;
+    flat_entry(fb, u, lb);
+    const int si = u / n;
+    const EbAdjEnt &E = tab[u - si * n];
+    int q = -s0;
+    ((q++ == si ? adj_block<S>(E, lb, hc, dtp) : (void)0), ...);
+}
+
+// The stages [s0, s1) of the list, kGridRows entries to a launch (grid.y,
+// where the entries are too many to be flattened).
+template <int... S>
+void launch_adj_group(const EbAdjEnt *tab, const EbAdjEnt *htab, int n, const HydroConst &hc,
+                      const double *dtp, hipStream_t st, Prof *prof, int s0 = 0,
+                      int s1 = (int)sizeof...(S)) {
+    typedef int64_t (*Count)(const EbAdjEnt &);
+    const Count counts[] = {adj_blocks<S>...};
+    constexpr int stages[] = {S...};
+    const int per = kGridRows / (s1 - s0);
+    for (int b0 = 0; b0 < n; b0 += per) {
+        const int m = std::min(per, n - b0);
+        FlatBlocks fb;
+        const dim3 grid = flat_blocks(
+            (s1 - s0) * m, [&](int u) { return counts[s0 + u / m](htab[b0 + u % m]); }, fb);
+        if (grid.x == 0) continue;
+        Region reg(prof, adj_name(stages[s0]), st);
+        hipLaunchKernelGGL((k_eb_adj_sites<S...>), grid, dim3(kBlock), 0, st, tab + b0, m, s0, hc,
+                           dtp, fb);
+    }
+}
+
+// The stages in reverse order, independent ones in one launch (12 launches
+// where one per stage took 32; boxes whose pairs share a buffer go pair by
+// pair).
+void launch_all_adj(const EbAdjEnt *tab, const EbAdjEnt *htab, int n, const HydroConst &hc,
+                    const double *dtp, hipStream_t st, Prof *prof, const CutCell *cells,
+                    int ncells) {
+#define CAMR_EB_GO(...) launch_adj_group<__VA_ARGS__>(tab, htab, n, hc, dtp, st, prof)
+    auto final_solves = [&](int s0, int s1) {
+        launch_adj_group<AS_FINAL + 0, AS_FINAL + 2, AS_FINAL + 4, AS_DIVU>(tab, htab, n, hc, dtp,
+                                                                            st, prof, s0, s1);
+    };
+    auto final_states = [&](int s0, int s1) {
+        launch_adj_group<AS_FINAL + 1, AS_FINAL + 3, AS_FINAL + 5>(tab, htab, n, hc, dtp, st, prof,
+                                                                   s0, s1);
+    };
+    auto pair_solves = [&](int s0, int s1) {
+        launch_adj_group<AS_PAIR + 0, AS_PAIR + 2, AS_PAIR + 4, AS_PAIR + 6, AS_PAIR + 8,
+                         AS_PAIR + 10>(tab, htab, n, hc, dtp, st, prof, s0, s1);
+    };
+    auto pair_states = [&](int s0, int s1) {
+        launch_adj_group<AS_PAIR + 1, AS_PAIR + 3, AS_PAIR + 5, AS_PAIR + 7, AS_PAIR + 9,
+                         AS_PAIR + 11>(tab, htab, n, hc, dtp, st, prof, s0, s1);
+    };
+    CAMR_EB_GO(AS_RDST);
+    if (!cells) {
+        CAMR_EB_GO(AS_RSRC);
+        CAMR_EB_GO(AS_DIVCUT);
+    } else if (ncells > 0) {
+        {
+            Region reg(prof, adj_name(AS_RSRC), st);
+            hipLaunchKernelGGL(k_eb_adj_list<AS_RSRC>, dim3(grid_for(ncells), NH), dim3(kBlock), 0,
+                               st, tab, cells, ncells, hc);
+        }
+        Region reg(prof, adj_name(AS_DIVCUT), st);
+        hipLaunchKernelGGL(k_eb_adj_list<AS_DIVCUT>, dim3(grid_for(ncells), NH + 2), dim3(kBlock),
+                           0, st, tab, cells, ncells, hc);
+    }
+    CAMR_EB_GO(AS_DIV);
+    CAMR_EB_GO(AS_ADJ + 0, AS_ADJ + 1, AS_ADJ + 2);
+    if (htab[0].A.keep()) {
+        final_solves(0, 4);
+        final_states(0, 3);
+        pair_solves(0, 6);
+        pair_states(0, 6);
+    } else {
+        final_solves(3, 4);
+        for (int d = 0; d < 3; ++d) { final_solves(d, d + 1); final_states(d, d + 1); }
+        for (int p = 0; p < 6; ++p) { pair_solves(p, p + 1); pair_states(p, p + 1); }
+    }
+    CAMR_EB_GO(AS_R1 + 0, AS_R1 + 1, AS_R1 + 2);
+    CAMR_EB_GO(AS_PLM);
+    CAMR_EB_GO(AS_PRIM);
+#undef CAMR_EB_GO
 }
 
 __device__ __forceinline__ bool batch_pt(const DevFab *tab, int g, int &b, int &i, int &j,
@@ -975,8 +1062,7 @@ int eb_adjoint_batch(const EbAdjEnt *tab, const EbAdjEnt *htab, int n, const Hyd
                      const double *dtp, hipStream_t st, Prof *prof, const CutCell *cells,
                      int ncells) {
     if (n <= 0) return CAMR_OK;
-    launch_adjs(std::make_integer_sequence<int, AS_COUNT>{}, tab, htab, n, hc, dtp, st, prof,
-                cells, ncells);
+    launch_all_adj(tab, htab, n, hc, dtp, st, prof, cells, ncells);
     return hipGetLastError() == hipSuccess ? CAMR_OK : CAMR_ERR_HIP;
 }
 
