@@ -26,6 +26,7 @@
 #include "hydro_adjoint.h"
 #include "hydro_eb_adjoint.h"
 #include "hydro_fused.h"
+#include "hydro_mol.h"
 #include "hydro_state.h"
 
 namespace camr {
@@ -311,6 +312,9 @@ class HydroLevel {
     // cleaned: src went through clean_all (kb_expand_cleaned, one pass)
     void expand_all(const DevFab *src, bool cleaned = false);
     int hydro_on_workers(double dt);
+    // method of lines, engine 0: the hydro source of every box in four
+    // launches (not with flux registers, which need the face fluxes)
+    MolEngine mol_;
     // staged engine: the step captured once per buffer parity, replayed
     // with the step's dt in dt_dev_
     // [buffer parity][post_timestep clean deferred]
@@ -925,6 +929,10 @@ int HydroLevel::create() {
             sc = std::max(sc, desc_.hp.do_mol ? umdrv_mol_scratch_doubles(B)
                                               : umdrv_staged_scratch_doubles(B));
         if ((rc = setup_workers(max_g4, sc))) return rc;
+        if (desc_.hp.do_mol && desc_.engine == 0 &&
+            std::all_of(box_.begin(), box_.end(), MolEngine::fits) &&
+            (rc = mol_.setup(box_, sbv_, dsv_)))
+            return rc;
     }
     return CAMR_OK;
 }
@@ -1829,6 +1837,8 @@ void HydroLevel::expand_all(const DevFab *src, bool cleaned) {
 // construct_hydro_source into dSdt of every box, spread over the worker
 // streams between a fork and a join.
 int HydroLevel::hydro_on_workers(double dt) {
+    if (mol_.ready() && !reg_crse_ && !reg_fine_)
+        return mol_.source(hc_, stream_, status_, &prof_);
     int rc = fork();
     if (rc) return rc;
     in_ws_ = true;

@@ -582,37 +582,6 @@ __device__ __forceinline__ void trans2_point(const Batch &B, int w, int nw, cons
 // instead of a second load of the plane below.  Same per-point arithmetic
 // as k_trans1<2> / k_trans2<2, S>, hence the same results.
 
-// adjust_face<D> (hydro_artif_visc, hydro_norm_spec_flx, hydro_ext_flx) on
-// values: d4 the face's four nodal divergences in adjust_face's order (the
-// face's node, +e_T0, +e_T1, +e_T0+e_T1); uc/um the conserved state of the
-// cells above and below the face.
-template <int D>
-__device__ __forceinline__ void adjust_face_vals(double *f, const double *d4,
-                                                 const double *uc, const double *um, int idx,
-                                                 double area, const HydroConst &hc) {
-    const double div = hc.difmag * vmin(0.0, 0.25 * (d4[0] + d4[1] + d4[2] + d4[3]));
-    const bool at_bndry = (idx == hc.domlo[D] && hc.bclo[D] == BC_NOSLIPWALL) ||
-                          (idx == hc.domhi[D] + 1 && hc.bchi[D] == BC_NOSLIPWALL);
-    const double dxd = hc.dx[D];
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n) {
-        if (n == UTEMP) continue;
-        const bool tang = (n == UMX || n == UMY || n == UMZ) && (n != UMX + D);
-        if (!(at_bndry && tang)) f[n] += dxd * div * (uc[n] - um[n]);
-    }
-    f[UTEMP] = 0.0;
-    double summ = 0.0;
-    summ += f[UFS];
-    summ += f[UFS + 1];
-    summ += f[UFS + 2];
-    const double fac = (summ != 0.0) ? f[URHO] / summ : 1.0;
-    f[UFS] *= fac;
-    f[UFS + 1] *= fac;
-    f[UFS + 2] *= fac;
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n) f[n] *= area;
-}
-
 // transdo differences of the cell at offset v in direction T (faces v and
 // v + e_T of F)
 template <int T>

@@ -142,4 +142,45 @@ CAMR_HD void adjust_face(double *f, const DA &divu,
     for (int n = 0; n < NVAR; ++n) f[n] *= area;
 }
 
+// adjust_face<D> (hydro_artif_visc, hydro_norm_spec_flx, hydro_ext_flx) on
+// values: dsum the sum of the face's four nodal divergences in adjust_face's
+// order (the face's node, +e_T0, +e_T1, +e_T0+e_T1); du the conserved state of
+// the cell above the face minus that of the one below.
+template <int D>
+__device__ __forceinline__ void adjust_face_jump(double *f, double dsum, const double *du, int idx,
+                                                 double area, const HydroConst &hc) {
+    const double div = hc.difmag * vmin(0.0, 0.25 * dsum);
+    const bool at_bndry = (idx == hc.domlo[D] && hc.bclo[D] == BC_NOSLIPWALL) ||
+                          (idx == hc.domhi[D] + 1 && hc.bchi[D] == BC_NOSLIPWALL);
+    const double dxd = hc.dx[D];
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) {
+        if (n == UTEMP) continue;
+        const bool tang = (n == UMX || n == UMY || n == UMZ) && (n != UMX + D);
+        if (!(at_bndry && tang)) f[n] += dxd * div * du[n];
+    }
+    f[UTEMP] = 0.0;
+    double summ = 0.0;
+    summ += f[UFS];
+    summ += f[UFS + 1];
+    summ += f[UFS + 2];
+    const double fac = (summ != 0.0) ? f[URHO] / summ : 1.0;
+    f[UFS] *= fac;
+    f[UFS + 1] *= fac;
+    f[UFS + 2] *= fac;
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) f[n] *= area;
+}
+
+// The same from the divergences and the states above and below (uc, um).
+template <int D>
+__device__ __forceinline__ void adjust_face_vals(double *f, const double *d4,
+                                                 const double *uc, const double *um, int idx,
+                                                 double area, const HydroConst &hc) {
+    double du[NVAR];
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) du[n] = n == UTEMP ? 0.0 : uc[n] - um[n];
+    adjust_face_jump<D>(f, d4[0] + d4[1] + d4[2] + d4[3], du, idx, area, hc);
+}
+
 } // namespace camr

@@ -213,7 +213,9 @@ typedef struct camr_level_desc {
     const int32_t *box_lohi; /* host array of nbox*6 ints: lo[3], hi[3] */
     int32_t engine;          /* 0 = fused, or staged for boxes too large for the fused
                                 engine's 32-bit layout (default); 1 = staged per-stage
-                                kernels; 2 = fused only */
+                                kernels; 2 = fused only.  The method of lines: 0 =
+                                its hydro source in four launches over every box
+                                (per stage with flux registers), 1 = per stage */
     int32_t batched;         /* fused engine: 1 = each stage is one launch over every
                                 box of the level (default); 0 = one launch per box,
                                 the per-box loop of construct_hydro_source
