@@ -329,8 +329,7 @@ class HydroLevel {
     double *ext_ = nullptr;     // exterior data (whole domain), when set
     double *cstage_ = nullptr;  // coarse values staged for exterior_from
     size_t cstage_n_ = 0;
-    // the domain cells, in domain order, that the boxes' ghost regions map
-    // to and no box owns (x, y, z triples; built on the first ghost fill)
+    // the domain cells that the boxes' ghost regions map to and no box owns (x, y, z triples; built on the first ghost fill)
     int *shell_cells_ = nullptr;
     int64_t shell_n_ = -1;
     // the coarse cells (grown coarse domain) their interpolation reads, for
@@ -414,7 +413,7 @@ class HydroLevel {
     }
     int set_exterior(const double *h);
     int exterior_from(HydroLevel &coarse, int ratio, int tmode = 0, double ta = 0.0,
-                      double tb = 0.0, bool ghosts_only = false);
+                      double tb = 0.0);
     int set_tuning(const Tuning &t);
     int get_tuning(Tuning *t) const;
     bool fused() const { return fused_; }
@@ -496,10 +495,9 @@ int HydroLevel::set_exterior(const double *h) {
 }
 
 // Exterior data from the coarser level: FillPatch's coarse-fine
-// interpolation (k_ext_from_coarse) at every cell of this level's domain,
-// from the coarse level's current S_new.
-int HydroLevel::exterior_from(HydroLevel &C, int ratio, int tmode, double ta, double tb,
-                              bool ghosts_only) {
+// interpolation (k_ext_cells) at the cells that this level's ghost fills
+// read, from the coarse level's current S_new.
+int HydroLevel::exterior_from(HydroLevel &C, int ratio, int tmode, double ta, double tb) {
     if (ratio < 2) { set_error("refinement ratio must be at least 2"); return CAMR_ERR_PARAM; }
     // EB builds interpolate with eb_cell_cons_interp (CAMR_setup.cpp:139-143),
     // which weighs by volume fractions and skips covered cells: not built
@@ -536,35 +534,23 @@ int HydroLevel::exterior_from(HydroLevel &C, int ratio, int tmode, double ta, do
         cstage_n_ = NVAR * cst.npts();
     }
     const Arr stv = dense(cstage_, cst);
-    if (ghosts_only) {
-        // just the cells a fill reads from the exterior: the domain images
-        // of the boxes' ghost regions that no box owns, and the coarse
-        // cells their interpolation reads
-        if (shell_n_ < 0 || shell_ratio_ != ratio) {
-            rc = build_shell_cells(ratio, make_box(C.desc_.hp.domlo, C.desc_.hp.domhi));
-            if (rc) return rc;
-        }
-        if (cstage_cells_n_ > 0)
-            hipLaunchKernelGGL(k_coarse_stage_cells, dim3(grid_for(cstage_cells_n_), NVAR),
-                               dim3(kBlock), 0, stream_, (const int *)cstage_cells_,
-                               cstage_cells_n_, stv, ct, (const int *)C.owner_, C.dom_, co, tmode,
-                               ta, tb);
-        // pass 2: one thread per fine cell and component (grid.y = NVAR)
-        if (shell_n_ > 0)
-            hipLaunchKernelGGL(k_ext_cells, dim3(grid_for(shell_n_), NVAR), dim3(kBlock), 0,
-                               stream_, (const int *)shell_cells_, shell_n_, extv_, stv, C.dom_,
-                               ratio, dom.lo[0], dom.lo[1], dom.lo[2]);
-    } else {
-        {
-            const Range r = range_of(cst);
-            hipLaunchKernelGGL(k_coarse_stage, dim3(grid_for(r.n), NVAR), dim3(kBlock), 0, stream_,
-                               r, stv, ct, (const int *)C.owner_, C.dom_, co, tmode, ta, tb);
-        }
-        const Range r = range_of(dom);
-        hipLaunchKernelGGL(k_ext_from_coarse, dim3(grid_for(r.n), NVAR), dim3(kBlock), 0, stream_,
-                           r, extv_, stv, C.dom_, ratio, dom.lo[0], dom.lo[1], dom.lo[2],
-                           (const int *)nullptr, dom_);
+    // just the cells a fill reads from the exterior: the domain images of the
+    // boxes' ghost regions that no box owns, and the coarse cells their
+    // interpolation reads (boxes over a sphere's shell of a 128^3 domain: 39 us
+    // of k_ext_cells and staging; all of the domain 400)
+    if (shell_n_ < 0 || shell_ratio_ != ratio) {
+        rc = build_shell_cells(ratio, make_box(C.desc_.hp.domlo, C.desc_.hp.domhi));
+        if (rc) return rc;
     }
+    if (cstage_cells_n_ > 0)
+        hipLaunchKernelGGL(k_coarse_stage_cells, dim3(grid_for(cstage_cells_n_), NVAR),
+                           dim3(kBlock), 0, stream_, (const int *)cstage_cells_, cstage_cells_n_,
+                           stv, ct, (const int *)C.owner_, C.dom_, co, tmode, ta, tb);
+    // pass 2: one thread per fine cell and component (grid.y = NVAR)
+    if (shell_n_ > 0)
+        hipLaunchKernelGGL(k_ext_cells, dim3(grid_for(shell_n_), NVAR), dim3(kBlock), 0, stream_,
+                           (const int *)shell_cells_, shell_n_, extv_, stv, C.dom_, ratio,
+                           dom.lo[0], dom.lo[1], dom.lo[2]);
     CAMR_HIP(hipGetLastError());
     // the coarse level may step next: finish reading its state first
     CAMR_HIP(hipStreamSynchronize(stream_));
@@ -580,75 +566,57 @@ void HydroLevel::drop_shell_cells() {
     shell_ratio_ = 0;
 }
 
+// The lists are made on the device: marks, then the marked cells counted and
+// written.  (By a host loop over the grown boxes and the domain they were half
+// of the first pass of a 96^3 level with a refined block in it: 15.5 ms, now
+// 7.0.)  Their order is that of the atomics, so only the cells' grouping into
+// blocks varies.
 int HydroLevel::build_shell_cells(int ratio, const Box &cdom) {
     drop_shell_cells();
-    const Box dom = make_box(desc_.hp.domlo, desc_.hp.domhi);
-    const int64_t n0 = dom.len(0), n1 = dom.len(1), n2 = dom.len(2);
-    std::vector<int> own((size_t)dom.npts());
-    CAMR_HIP(hipMemcpy(own.data(), owner_, own.size() * sizeof(int), hipMemcpyDeviceToHost));
-    std::vector<uint8_t> mark(own.size(), 0);
-    const int64_t len[3] = {n0, n1, n2};
-    for (const Box &B0 : box_) {
-        const Box G = grow(B0, ng_);
-        for (int k = G.lo[2]; k <= G.hi[2]; ++k)
-            for (int j = G.lo[1]; j <= G.hi[1]; ++j)
-                for (int i = G.lo[0]; i <= G.hi[0]; ++i) {
-                    const int c[3] = {i, j, k};
-                    int64_t m[3];
-                    bool in = true;
-                    for (int d = 0; d < 3 && in; ++d) {
-                        int64_t x = c[d] - dom.lo[d];
-                        if (x < 0 || x >= len[d]) {
-                            if (!desc_.is_periodic[d]) in = false;
-                            else x = (x % len[d] + len[d]) % len[d];
-                        }
-                        m[d] = x;
-                    }
-                    if (!in) continue;
-                    const int64_t at = m[0] + m[1] * n0 + m[2] * n0 * n1;
-                    if (own[(size_t)at] < 0) mark[(size_t)at] = 1;
-                }
+    const Box dom = make_box(desc_.hp.domlo, desc_.hp.domhi), cst = grow(cdom, 1);
+    const Range rd = range_of(dom), rc = range_of(cst);
+    uint8_t *mark = nullptr;  // of the fine domain, then of the staged box
+    int *count = nullptr;
+    CAMR_HIP(hipMalloc(&mark, (size_t)(rd.n + rc.n)));
+    hipError_t e = hipMalloc(&count, 2 * sizeof(int));
+    auto list = [&](const Range &r, const uint8_t *m, int *cnt, int **cells, int64_t *n) {
+        int h = 0;
+        hipLaunchKernelGGL(k_list_marked, dim3(grid_for(r.n)), dim3(kBlock), 0, stream_, r, m, cnt,
+                           (int *)nullptr);
+        hipError_t q = hipMemcpyAsync(&h, cnt, sizeof(int), hipMemcpyDeviceToHost, stream_);
+        if (q == hipSuccess) q = hipStreamSynchronize(stream_);
+        *n = h;
+        if (q != hipSuccess || h == 0) return q;
+        q = hipMalloc(cells, (size_t)3 * h * sizeof(int));
+        if (q != hipSuccess) return q;
+        hipLaunchKernelGGL(k_fill_bytes, dim3(1), dim3(64), 0, stream_, (uint8_t *)cnt,
+                           (int64_t)sizeof(int));
+        hipLaunchKernelGGL(k_list_marked, dim3(grid_for(r.n)), dim3(kBlock), 0, stream_, r, m, cnt,
+                           *cells);
+        return hipGetLastError();
+    };
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_fill_bytes, dim3(grid_for(rd.n + rc.n)), dim3(kBlock), 0, stream_, mark,
+                           rd.n + rc.n);
+        hipLaunchKernelGGL(k_fill_bytes, dim3(1), dim3(64), 0, stream_, (uint8_t *)count,
+                           (int64_t)(2 * sizeof(int)));
+        launch_all(kb_mark_shell, ng_, (const DevFab *)tab_a_, ng_, (const int *)owner_, dom_, mark);
+        // the coarse parents of the marked cells and their 26 neighbours,
+        // over the coarse domain grown by one (the staged array's box)
+        hipLaunchKernelGGL(k_mark_parents, dim3(grid_for(rd.n)), dim3(kBlock), 0, stream_, rd,
+                           (const uint8_t *)mark, ratio, rc, mark + rd.n);
+        int64_t nf = 0;
+        e = list(rd, mark, count, &shell_cells_, &nf);
+        if (e == hipSuccess) e = list(rc, mark + rd.n, count + 1, &cstage_cells_, &cstage_cells_n_);
+        shell_n_ = nf;
+        if (e == hipSuccess) e = hipStreamSynchronize(stream_);
     }
-    // the coarse parents of the listed cells and their 26 neighbours, over
-    // the coarse domain grown by one (the staged array's box)
-    const Box cst = grow(cdom, 1);
-    const int64_t c0 = cst.len(0), c1 = cst.len(1), c2 = cst.len(2);
-    std::vector<uint8_t> cmark((size_t)cst.npts(), 0);
-    std::vector<int> cells;
-    for (int64_t k = 0; k < n2; ++k)
-        for (int64_t j = 0; j < n1; ++j)
-            for (int64_t i = 0; i < n0; ++i)
-                if (mark[(size_t)(i + j * n0 + k * n0 * n1)]) {
-                    cells.push_back((int)i + dom.lo[0]);
-                    cells.push_back((int)j + dom.lo[1]);
-                    cells.push_back((int)k + dom.lo[2]);
-                    // parent in the staged box's index space (cst.lo = cdom.lo - 1)
-                    const int64_t pi = i / ratio + 1, pj = j / ratio + 1, pk = k / ratio + 1;
-                    for (int64_t dk = -1; dk <= 1; ++dk)
-                        for (int64_t dj = -1; dj <= 1; ++dj)
-                            for (int64_t di = -1; di <= 1; ++di)
-                                cmark[(size_t)((pi + di) + (pj + dj) * c0 + (pk + dk) * c0 * c1)] = 1;
-                }
-    shell_n_ = (int64_t)(cells.size() / 3);
-    if (shell_n_ > 0) {
-        CAMR_HIP(hipMalloc(&shell_cells_, cells.size() * sizeof(int)));
-        CAMR_HIP(hipMemcpy(shell_cells_, cells.data(), cells.size() * sizeof(int),
-                           hipMemcpyHostToDevice));
-    }
-    std::vector<int> ccells;
-    for (int64_t k = 0; k < c2; ++k)
-        for (int64_t j = 0; j < c1; ++j)
-            for (int64_t i = 0; i < c0; ++i)
-                if (cmark[(size_t)(i + j * c0 + k * c0 * c1)]) {
-                    ccells.push_back((int)i + cst.lo[0]);
-                    ccells.push_back((int)j + cst.lo[1]);
-                    ccells.push_back((int)k + cst.lo[2]);
-                }
-    cstage_cells_n_ = (int64_t)(ccells.size() / 3);
-    if (cstage_cells_n_ > 0) {
-        CAMR_HIP(hipMalloc(&cstage_cells_, ccells.size() * sizeof(int)));
-        CAMR_HIP(hipMemcpy(cstage_cells_, ccells.data(), ccells.size() * sizeof(int),
-                           hipMemcpyHostToDevice));
+    (void)hipFree(mark);
+    (void)hipFree(count);
+    if (e != hipSuccess) {
+        drop_shell_cells();
+        set_error("coarse-fine ghost list: %s", hipGetErrorString(e));
+        return CAMR_ERR_HIP;
     }
     shell_ratio_ = ratio;
     return CAMR_OK;
@@ -3016,7 +2984,7 @@ int amr_advance_level(const std::vector<HydroLevel *> &L, const std::vector<Flux
         if (t > t_old - teps && t < t_old + teps) tmode = 1;
         else if (t > t_new - teps && t < t_new + teps) tmode = 0;
         const double ta = (t_new - t) / (t_new - t_old), tb = (t - t_old) / (t_new - t_old);
-        if ((rc = F.exterior_from(C, Rg.ratio, tmode, ta, tb, true))) return rc;
+        if ((rc = F.exterior_from(C, Rg.ratio, tmode, ta, tb))) return rc;
         if ((rc = amr_advance_level(L, R, l + 1, dtf))) return rc;
     }
     if ((rc = F.resolve())) return rc;

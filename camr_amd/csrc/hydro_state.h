@@ -118,13 +118,9 @@ __global__ void kb_tail_redo(const DevFab *snew, const DevFab *sb, const DevFab 
                              const DevFab *dsdt, int nbox, const double *dtp, double g,
                              int add_grav, int post, int mol, HydroConst hc, int *flags,
                              int *redo, EbFlags eb, unsigned long long *dtmin);
-__global__ void k_coarse_stage(Range r, Arr st, const DevFab *ctab, const int *cowner, DomInfo CD,
-                               const DevFab *otab, int tmode, double ta, double tb);
 __global__ void k_coarse_stage_cells(const int *cells, int64_t ncells, Arr st, const DevFab *ctab,
                                      const int *cowner, DomInfo CD, const DevFab *otab, int tmode,
                                      double ta, double tb);
-__global__ void k_ext_from_coarse(Range r, Arr ext, Arr st, DomInfo CD, int ratio, int flo0,
-                                  int flo1, int flo2, const int *fowner, DomInfo FD);
 __global__ void k_ext_cells(const int *cells, int64_t ncells, Arr ext, Arr st, DomInfo CD,
                             int ratio, int flo0, int flo1, int flo2);
 // coarse-fine synchronisation (flux register, reflux, average_down)
@@ -161,5 +157,11 @@ inline void launch_on(K kern, const Box &b, hipStream_t s, A... args) {
     Range r = range_of(b);
     hipLaunchKernelGGL(kern, dim3(grid_for(r.n)), dim3(kBlock), 0, s, r, args...);
 }
+
+__global__ void k_fill_bytes(uint8_t *p, int64_t n);
+__global__ void kb_mark_shell(const DevFab *tab, int ng, const int *owner, DomInfo D,
+                              uint8_t *mark);
+__global__ void k_mark_parents(Range rd, const uint8_t *mark, int ratio, Range rc, uint8_t *cmark);
+__global__ void k_list_marked(Range r, const uint8_t *mark, int *count, int *cells);
 
 } // namespace camr

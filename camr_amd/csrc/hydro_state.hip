@@ -970,8 +970,8 @@ kb_avgdown(const DevFab *csnew, const DevFab *ftab, const int *fowner, DomInfo F
 // coarse data, then one factor alpha in [0,1] for the slope vector so that
 // every child lies within the min / max of the 27 coarse neighbours, into
 // the fine level's exterior array.  Two passes: the coarse values staged
-// densely (k_coarse_stage*), then one thread per fine cell and component
-// (k_ext_*).
+// densely (k_coarse_stage_cells), then one thread per fine cell and component
+// (k_ext_cells), both over lists of the cells that ghost fills need.
 
 // The coarse value FillPatch sees at (i, j, k), components [nlo, nhi):
 // its source cell through the domain's periodicity / BCs, at the fill
@@ -1000,18 +1000,8 @@ __device__ __forceinline__ void stage_point(int i, int j, int k, const Arr &st, 
     }
 }
 
-__global__ void __launch_bounds__(kBlock)
-k_coarse_stage(Range r, Arr st, const DevFab *ctab, const int *cowner, DomInfo CD,
-               const DevFab *otab, int tmode, double ta, double tb) {
-    int i, j, k;
-    if (!range_point(r, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, i, j, k)) return;
-    const int nlo = gridDim.y > 1 ? (int)blockIdx.y : 0;
-    const int nhi = gridDim.y > 1 ? (int)blockIdx.y + 1 : NVAR;
-    stage_point(i, j, k, st, ctab, cowner, CD, otab, tmode, ta, tb, nlo, nhi);
-}
-
-// The same staging over a list of coarse cells (x, y, z triples), one
-// component per block row.
+// The staging over a list of coarse cells (x, y, z triples), one component
+// per block row.
 __global__ void __launch_bounds__(kBlock)
 k_coarse_stage_cells(const int *cells, int64_t ncells, Arr st, const DevFab *ctab,
                      const int *cowner, DomInfo CD, const DevFab *otab, int tmode, double ta,
@@ -1029,28 +1019,71 @@ __device__ __forceinline__ void ext_point(int i, int j, int k, const Arr &ext, c
                                           const DomInfo &CD, int ratio, const int *flo, int nlo,
                                           int nhi);
 
+// ---- lists of the cells above: marks, then the marked cells of a range
 __global__ void __launch_bounds__(kBlock)
-k_ext_from_coarse(Range r, Arr ext, Arr st, DomInfo CD, int ratio, int flo0, int flo1, int flo2,
-                  const int *fowner, DomInfo FD) {
-    int i, j, k;
-    if (!range_point(r, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, i, j, k)) return;
-    if (fowner) {
-        // ghost-shell mode: r is a grown fine box; take the cell's domain
-        // image and skip it when outside a non-periodic domain or owned
-        int c[3] = {i, j, k}, m[3];
-        if (!reg_map(FD, c, m) || owner_of(FD, fowner, m) >= 0) return;
-        i = m[0];
-        j = m[1];
-        k = m[2];
-    }
-    const int flo[3] = {flo0, flo1, flo2};
-    // grid.y > 1: one component per block row
-    const int nlo = gridDim.y > 1 ? (int)blockIdx.y : 0;
-    const int nhi = gridDim.y > 1 ? (int)blockIdx.y + 1 : NVAR;
-    ext_point(i, j, k, ext, st, CD, ratio, flo, nlo, nhi);
+k_fill_bytes(uint8_t *p, int64_t n) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < n) p[t] = 0;
 }
 
-// The same interpolation over a list of fine cells (x, y, z triples, each
+// The domain images of the boxes' ghost cells that no box owns.
+__global__ void __launch_bounds__(kBlock)
+kb_mark_shell(const DevFab *tab, int ng, const int *owner, DomInfo D, uint8_t *mark) {
+    int c[3], m[3];
+    if (!range_point(range_of(grow(tab[blockIdx.y].b, ng)),
+                     (int64_t)blockIdx.x * blockDim.x + threadIdx.x, c[0], c[1], c[2]))
+        return;
+    if (!reg_map(D, c, m)) return;
+    const int64_t n0 = D.domhi[0] - D.domlo[0] + 1, n1 = D.domhi[1] - D.domlo[1] + 1;
+    const int64_t at = (m[0] - D.domlo[0]) + (m[1] - D.domlo[1]) * n0 + (m[2] - D.domlo[2]) * n0 * n1;
+    if (owner[at] < 0) mark[at] = 1;
+}
+
+// Marks in range rc (the coarse domain grown by one) the parents of the
+// marked cells of the fine domain rd and the parents' 26 neighbours.
+__global__ void __launch_bounds__(kBlock)
+k_mark_parents(Range rd, const uint8_t *mark, int ratio, Range rc, uint8_t *cmark) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int i, j, k;
+    if (!range_point(rd, t, i, j, k) || !mark[t]) return;
+    const int64_t pi = (i - rd.lo0) / ratio, pj = (j - rd.lo1) / ratio, pk = (k - rd.lo2) / ratio;
+    for (int64_t dk = 0; dk <= 2; ++dk)
+        for (int64_t dj = 0; dj <= 2; ++dj)
+            for (int64_t di = 0; di <= 2; ++di)
+                cmark[(pi + di) + (pj + dj) * rc.n0 + (pk + dk) * (int64_t)rc.n0 * rc.n1] = 1;
+}
+
+// Adds the marked cells of r to *count and, with cells, writes them there
+// (x, y, z triples), a block's together: one atomic add per block.
+__global__ void __launch_bounds__(kBlock)
+k_list_marked(Range r, const uint8_t *mark, int *count, int *cells) {
+    __shared__ int at[kBlock / 64];
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int i = 0, j = 0, k = 0;
+    const bool m = range_point(r, t, i, j, k) && mark[t];
+    const unsigned long long ballot = __ballot(m);
+    const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
+    if (lane == 0) at[wave] = __popcll(ballot);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int n = 0;
+        for (int w = 0; w < kBlock / 64; ++w) n += at[w];
+        int base = n ? atomicAdd(count, n) : 0;
+        for (int w = 0; w < kBlock / 64; ++w) {
+            const int x = at[w];
+            at[w] = base;
+            base += x;
+        }
+    }
+    __syncthreads();
+    if (!m || !cells) return;
+    int *c = cells + 3 * ((int64_t)at[wave] + __popcll(ballot & ((1ull << lane) - 1)));
+    c[0] = i;
+    c[1] = j;
+    c[2] = k;
+}
+
+// The interpolation over a list of fine cells (x, y, z triples, each
 // a domain cell no box owns), one component per block row.
 __global__ void __launch_bounds__(kBlock)
 k_ext_cells(const int *cells, int64_t ncells, Arr ext, Arr st, DomInfo CD, int ratio, int flo0,

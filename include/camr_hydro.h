@@ -262,9 +262,10 @@ int camr_level_set_exterior(camr_level *L, const double *host);
  * current state: FillPatch's coarse-to-fine interpolation (AmrLevel::
  * FillPatch, CAMR.cpp:1247, with the State_Type interpolater cell_cons_interp,
  * Source/Utils/CAMR_setup.cpp:141-144: conservative linear, MC-limited,
- * linearly limited) at every cell of the fine domain.  The fine domain must
- * be the coarse domain refined by `ratio`.  Single time level: the coarse
- * data of the moment (no time interpolation between coarse old and new). */
+ * linearly limited) at every cell that the fine level's ghost regions read.
+ * The fine domain must be the coarse domain refined by `ratio`.  Single time
+ * level: the coarse data of the moment (no time interpolation between coarse
+ * old and new). */
 int camr_level_exterior_from_coarse(camr_level *fine, camr_level *coarse, int32_t ratio);
 
 /*
