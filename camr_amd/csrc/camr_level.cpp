@@ -1829,9 +1829,7 @@ int HydroLevel::advance_fused(double dt) {
     fa.has_ext = ext_ ? 1 : 0;
     fa.dom = dom_;
     fa.hc = hc_;
-    fa.dtp = dt_dev_;
     fa.g = desc_.const_grav;
-    fa.add_grav = desc_.add_grav_src;
     fa.src = grav_src_values_ ? engine_.grav_src() : SRC_NONE;
     PostArgs pa;
     pa.hc = hc_;
@@ -1920,9 +1918,7 @@ int HydroLevel::capture_graphs() {
         fa.has_ext = ext_ ? 1 : 0;
         fa.dom = dom_;
         fa.hc = hc_;
-        fa.dtp = dtp;
         fa.g = desc_.const_grav;
-        fa.add_grav = desc_.add_grav_src;
         fa.src = SRC_NONE;
         PostArgs pa;
         pa.hc = hc_;
@@ -2201,9 +2197,7 @@ int HydroLevel::adjoint_step(double dt, bool check) {
     fa.has_ext = 0;
     fa.dom = dom_;
     fa.hc = hc_;
-    fa.dtp = dt_dev_;
     fa.g = desc_.const_grav;
-    fa.add_grav = desc_.add_grav_src;
     fa.src = SRC_NONE;
     rc = engine_.fill(-1, parity(), fa, stream_, status_, &prof_);
     // the update itself is applied in registers by the post-pass adjoint

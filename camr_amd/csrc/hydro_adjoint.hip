@@ -105,14 +105,17 @@ __device__ __forceinline__ void take_tf_bar(double *Fb, size_t cs, size_t e, dou
 __global__ void __launch_bounds__(kBlock)
 k_post_adj(Batch B, AdjArgs a) {
     BATCH_POINT(ST_VALID)
-    (void)L;
-    const Arr snew = E.snew;
+    const Arr sold = E.sold;
     const Arr bin = a.sbar_in[E.id].a;
+    const CView u = cview(L, slot_ptr<S_U>(E), NVAR);
+    const unsigned v0 = L.off(i, j, k);
     // inputs of the two (three) energy resets: S_new after the update, which
-    // the recompute leaves to this kernel (S_new holds the filled state)
+    // the recompute leaves to this kernel
     double x0[NVAR], x1[NVAR], x2[NVAR];
 #pragma unroll
-    for (int n = 0; n < NVAR; ++n) x0[n] = snew(i, j, k, n);
+    for (int n = 0; n < NVAR; ++n) x0[n] = u.ld(v0, n);
+    if (a.add_grav)
+        new_values(x0, 0.0, *a.dtp, sold(i, j, k, URHO), sold(i, j, k, UMZ));
     update_values(E, i, j, k, a.hc, *a.dtp, x0);
     if (x0[URHO] == 0.) atomicOr(a.status, 1 << CAMR_ERR_ZERO_DENSITY);
     else if (x0[URHO] < a.hc.small_dens) atomicOr(a.status, kFloorFlag);

@@ -390,9 +390,7 @@ struct FillArgs {
     int has_ext;
     DomInfo dom;
     HydroConst hc;
-    const double *dtp;       // the step's dt (device)
     double g;
-    int add_grav;
     int src;  // SRC_*: what fill writes to S_SRCQ (SRC_ALL with zeros)
 };
 struct PostArgs {
@@ -404,6 +402,19 @@ struct PostArgs {
     int defer_post;  // 1: leave post_timestep's clean_state to the caller
 };
 
+// S_new of a valid cell before the update, with the gravity source: v its
+// Sborder values, plus dt times the old source (CAMR_advance.cpp:112-118).
+__device__ __forceinline__ void new_values(double *v, double g, double dt, double rho_old,
+                                           double rhow_old) {
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) {
+        double src = 0.0;
+        if (n == UMZ) src = g * rho_old;
+        else if (n == UEDEN) src = g * rhow_old;
+        v[n] += dt * src;
+    }
+}
+
 // Grid of one stage launch over a box set.
 struct LaunchCfg {
     Batch B;
@@ -412,8 +423,8 @@ struct LaunchCfg {
 };
 void launch_fill_fused(const LaunchCfg &c, const FillArgs &a, hipStream_t st, int *status);
 void launch_post_fused(const LaunchCfg &c, const PostArgs &a, hipStream_t st, int *status);
-// The update of k_update_c and the post pass in one kernel (S_new read and
-// written once).
+// S_new from the fill's Sborder copy (new_values), the update of k_update_c
+// and the post pass in one kernel (S_new only written).
 void launch_update_post_fused(const LaunchCfg &c, const HydroConst &hc, const double *dtp,
                               const PostArgs &a, hipStream_t st, int *status);
 

@@ -8,9 +8,9 @@
 //                              ghosts after normalize_species
 //   hydro_ctoprim              (CAMR_construct_hydro_source.cpp:108-120)
 //   hydro_srctoprim of a constant gravity's old source (:129-143)
+// k_update_post, one thread per valid cell:
 //   S_new = Sborder + dt * old source (CAMR_advance.cpp:112-118)
-// k_post_fused, one thread per valid cell, after S_new += dt dS/dt
-// (k_update_post: the update itself and then the same):
+//   S_new += dt dS/dt
 //   clean_state(S_new), new-source Saxpy, clean_state, post_timestep's
 //   clean_state (CAMR_advance.cpp:146-154; CAMR.cpp:698-699), then the
 //   CFL estimate of the next computeNewDt (Timestep.H:18-61).
@@ -22,10 +22,10 @@
 // Both are exact compositions of the reference's passes as long as no
 // density floor fires (enforce_min_density is the only non-pointwise piece;
 // normalize_species and the energy reset never change rho, rho*u):
-// k_fill_fused flags rho < small_dens in raw S_old, k_update_c flags it in
+// k_fill_fused flags rho < small_dens in raw S_old, k_update_post flags it in
 // S_new, and the level driver then recomputes the step with the unfused
 // sequence from the untouched raw S_old.  Both move at about the rate of a
-// copy (256^3: 6.0 GB in 1.32 ms and 9.4 GB in 1.70 ms).  Constant gravity
+// copy (256^3: 4.7 GB in 0.95 ms and 9.4 GB in 1.65 ms).  Constant gravity
 // takes the same two passes: 19 pass-by-pass launches of a 97x83x61 step
 // with gravity (0.34 of its 0.97 ms) became 2, 0.76 ms.
 #include "hydro_fused.h"
@@ -43,7 +43,7 @@ k_fill_fused(Batch B, FillArgs a, int *status) {
     const bool phys = map_cell(a.dom, i, j, k, m, &odd);
     const int ob = owner_of(a.dom, a.owner, m);
     double v[NVAR];
-    double rho_old = 0.0, rhow_old = 0.0;
+    double rho_old = 0.0;
     const bool valid = E.bx.contains(i, j, k);
     if (ob >= 0) {
         const Arr s = a.sold_tab[ob].a;
@@ -51,7 +51,6 @@ k_fill_fused(Batch B, FillArgs a, int *status) {
         for (int n = 0; n < NVAR; ++n) v[n] = s(m[0], m[1], m[2], n);
         if (valid) floor_detect(v[URHO], a.hc.small_dens, status);
         rho_old = v[URHO];
-        rhow_old = v[UMZ];
         // clean_state(S_old) on the source cell
         normalize_species(v);
         reset_e_and_T(v, a.hc);
@@ -95,21 +94,6 @@ k_fill_fused(Batch B, FillArgs a, int *status) {
                 for (int n = 0; n < NS; ++n)
                     if (n != SW) sq.st(v0, n, w[n]);
             }
-        }
-    }
-    if (valid) {
-        const double dt = *a.dtp;
-        const Arr snew = E.snew;
-#pragma unroll
-        for (int n = 0; n < NVAR; ++n) {
-            double x = v[n];
-            if (a.add_grav) {
-                double src = 0.0;
-                if (n == UMZ) src = a.g * rho_old;
-                else if (n == UEDEN) src = a.g * rhow_old;
-                x += dt * src;
-            }
-            snew(i, j, k, n) = x;
         }
     }
 }
@@ -172,9 +156,10 @@ k_post_fused(Batch B, PostArgs a, int *status) {
     block_min_commit(dtv, a.dtmin, status);
 }
 
-// k_update_c followed by k_post_fused, with S_new kept in registers in
-// between (the same arithmetic: S_new is rounded once by the update either
-// way).
+// new_values, k_update_c and k_post_fused, with S_new kept in registers in
+// between (the same arithmetic: S_new is rounded once by each either way).
+// Written by the fill and read back here it cost 1.3 GB at 256^3: fill 1.33 ->
+// 0.95 ms, this kernel 1.70 -> 1.65 ms.
 #ifdef CAMR_UPD_MINW
 #define UPD_BOUNDS __launch_bounds__(kBlock, CAMR_UPD_MINW)
 #else
@@ -189,9 +174,14 @@ k_update_post(Batch B, HydroConst hc, const double *dtp, PostArgs a, int *status
     double dtv = 1.7976931348623157e308;
     if (batch_point(B, E.bx, lblk, i, j, k)) {
         const Arr snew = E.snew;
+        const Arr sold = E.sold;
+        const CView u = cview(E.L, slot_ptr<S_U>(E), NVAR);
+        const unsigned v0 = E.L.off(i, j, k);
         double v[NVAR];
 #pragma unroll
-        for (int n = 0; n < NVAR; ++n) v[n] = snew(i, j, k, n);
+        for (int n = 0; n < NVAR; ++n) v[n] = u.ld(v0, n);
+        if (a.add_grav)
+            new_values(v, a.g, *dtp, sold(i, j, k, URHO), sold(i, j, k, UMZ));
         update_values(E, i, j, k, hc, *dtp, v);
         const double rho = v[URHO];
         if (rho == 0.) atomicOr(status, 1 << CAMR_ERR_ZERO_DENSITY);
