@@ -642,9 +642,13 @@ constexpr const char *site_name(int s) {
 }
 
 // The cut-cell divergence over a list of the cut cells, one component per
-// block row (grid.y = NVAR).  A few thousand cells are a handful of blocks,
-// so the time is one thread's chain of dependent loads: all ten components
-// in a thread took 110 us at 1.2e3 cells.
+// block row (grid.y = NVAR) or, from kCutPartCells on, all of them in a thread
+// (grid.y = 1).  A few thousand cells are a handful of blocks, so the time is
+// one thread's chain of dependent loads (2.9e3 cells: 25 us, all ten components
+// in a thread 110); with more of them it is the number of scattered loads, of
+// which the rows repeat the geometry's (9.6e3 cells of a 256x128x128 grid: 566
+// us, all in a thread 311).
+constexpr int kCutPartCells = 4096;
 __global__ void __launch_bounds__(kBlock)
 k_eb_divcut_list(const EbBox *tab, const CutCell *cells, int n, HydroConst hc) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -652,10 +656,10 @@ k_eb_divcut_list(const EbBox *tab, const CutCell *cells, int n, HydroConst hc) {
     const CutCell c = cells[t];
     const EbBox &B = tab[c.e];
     if (B.regular) return;  // no cut cell
-    const int m = (int)blockIdx.y;
+    const int n0 = (int)blockIdx.y, n1 = gridDim.y > 1 ? n0 + 1 : (int)NVAR;
     b_eb_div<true>(c.i, c.j, c.k, B.bx, B.FT[0], B.FT[1], B.FT[2], B.QE[0], B.QE[1], B.QE[2], B.g,
                    B.q, B.qaux, B.divc, B.wt, B.flx[0], B.flx[1], B.flx[2], hc, 1.0 / hc.dx[0],
-                   1.0 / hc.dx[1], 1.0 / hc.dx[2], !B.noflx, m, m + 1);
+                   1.0 / hc.dx[1], 1.0 / hc.dx[2], !B.noflx, n0, n1);
 }
 
 // The redistribution's source side over the cut cells of grow(bx, 1) in
@@ -696,12 +700,11 @@ k_eb_sites(const EbBox *tab, int n, int s0, HydroConst hc, const double *dtp, in
     ((q++ == si ? site_block<S>(B, lb, hc, dtp, has_src) : (void)0), ...);
 }
 
-// The sites [s0, s1) of the list, kGridRows entries to a launch (grid.y, where
-// the entries are too many to be flattened).
+// One launch over the entries of sites [s0, s1) of the list, kGridRows of them
+// to a launch (grid.y, where the entries are too many to be flattened).
 template <int... S>
-void launch_group(const EbBox *tab, const EbBox *htab, int n, const HydroConst &hc,
-                  const double *dtp, int has_src, hipStream_t st, Prof *prof, int s0 = 0,
-                  int s1 = (int)sizeof...(S)) {
+void launch_sites(const EbBox *tab, const EbBox *htab, int n, const HydroConst &hc,
+                  const double *dtp, int has_src, hipStream_t st, Prof *prof, int s0, int s1) {
     typedef int64_t (*Count)(const EbBox &);
     const Count counts[] = {site_blocks<S>...};
     constexpr int sites[] = {S...};
@@ -718,9 +721,29 @@ void launch_group(const EbBox *tab, const EbBox *htab, int n, const HydroConst &
     }
 }
 
-// hydro_umdrv_eb's stages in order, stages that are independent of each
-// other in one launch: 11 launches where one per stage took 32.  Boxes whose
-// pairs share a buffer (EbBox::keep) go pair by pair.
+// The sites [s0, s1) of the list, in one launch or one each (kStageMergeBlocks).
+template <int... S>
+void launch_group(const EbBox *tab, const EbBox *htab, int n, const HydroConst &hc,
+                  const double *dtp, int has_src, hipStream_t st, Prof *prof, int s0 = 0,
+                  int s1 = (int)sizeof...(S)) {
+    typedef int64_t (*Count)(const EbBox &);
+    const Count counts[] = {site_blocks<S>...};
+    int64_t blocks = 0;
+    for (int s = s0; s < s1; ++s)
+        for (int b = 0; b < n; ++b) blocks += counts[s](htab[b]);
+    if (blocks <= kStageMergeBlocks && s1 - s0 > 1) {
+        launch_sites<S...>(tab, htab, n, hc, dtp, has_src, st, prof, s0, s1);
+        return;
+    }
+    int q = 0;
+    ((q >= s0 && q < s1 ? launch_sites<S>(tab, htab, n, hc, dtp, has_src, st, prof, 0, 1) : (void)0,
+      ++q),
+     ...);
+}
+
+// hydro_umdrv_eb's stages in order, on small tables stages that are
+// independent of each other in one launch: 11 launches where one per stage
+// takes 32.  Boxes whose pairs share a buffer (EbBox::keep) go pair by pair.
 void launch_all_sites(const EbBox *tab, const EbBox *htab, int n, const HydroConst &hc,
                       const double *dtp, int has_src, hipStream_t st, Prof *prof,
                       const CutCell *cells, int ncells) {
@@ -764,7 +787,8 @@ void launch_all_sites(const EbBox *tab, const EbBox *htab, int n, const HydroCon
         const dim3 g(grid_for(ncells), NVAR);
         {
             Region reg(prof, site_name(ES_DIVCUT), st);
-            hipLaunchKernelGGL(k_eb_divcut_list, g, dim3(kBlock), 0, st, tab, cells, ncells, hc);
+            hipLaunchKernelGGL(k_eb_divcut_list, ncells < kCutPartCells ? g : dim3(g.x), dim3(kBlock),
+                               0, st, tab, cells, ncells, hc);
         }
         Region reg(prof, site_name(ES_RSRC), st);
         hipLaunchKernelGGL(k_eb_rsrc_list, g, dim3(kBlock), 0, st, tab, cells, ncells);

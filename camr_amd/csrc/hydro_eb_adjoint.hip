@@ -965,12 +965,11 @@ k_eb_adj_sites(const EbAdjEnt *tab, int n, int s0, HydroConst hc, const double *
     ((q++ == si ? adj_block<S>(E, lb, hc, dtp) : (void)0), ...);
 }
 
-// The stages [s0, s1) of the list, kGridRows entries to a launch (grid.y,
-// where the entries are too many to be flattened).
+// One launch over the entries of stages [s0, s1) of the list, kGridRows of
+// them to a launch (grid.y, where the entries are too many to be flattened).
 template <int... S>
-void launch_adj_group(const EbAdjEnt *tab, const EbAdjEnt *htab, int n, const HydroConst &hc,
-                      const double *dtp, hipStream_t st, Prof *prof, int s0 = 0,
-                      int s1 = (int)sizeof...(S)) {
+void launch_adj_sites(const EbAdjEnt *tab, const EbAdjEnt *htab, int n, const HydroConst &hc,
+                      const double *dtp, hipStream_t st, Prof *prof, int s0, int s1) {
     typedef int64_t (*Count)(const EbAdjEnt &);
     const Count counts[] = {adj_blocks<S>...};
     constexpr int stages[] = {S...};
@@ -987,9 +986,28 @@ void launch_adj_group(const EbAdjEnt *tab, const EbAdjEnt *htab, int n, const Hy
     }
 }
 
-// The stages in reverse order, independent ones in one launch (12 launches
-// where one per stage took 32; boxes whose pairs share a buffer go pair by
-// pair).
+// The stages [s0, s1) of the list, in one launch or one each (kStageMergeBlocks).
+template <int... S>
+void launch_adj_group(const EbAdjEnt *tab, const EbAdjEnt *htab, int n, const HydroConst &hc,
+                      const double *dtp, hipStream_t st, Prof *prof, int s0 = 0,
+                      int s1 = (int)sizeof...(S)) {
+    typedef int64_t (*Count)(const EbAdjEnt &);
+    const Count counts[] = {adj_blocks<S>...};
+    int64_t blocks = 0;
+    for (int s = s0; s < s1; ++s)
+        for (int b = 0; b < n; ++b) blocks += counts[s](htab[b]);
+    if (blocks <= kStageMergeBlocks && s1 - s0 > 1) {
+        launch_adj_sites<S...>(tab, htab, n, hc, dtp, st, prof, s0, s1);
+        return;
+    }
+    int q = 0;
+    ((q >= s0 && q < s1 ? launch_adj_sites<S>(tab, htab, n, hc, dtp, st, prof, 0, 1) : (void)0, ++q),
+     ...);
+}
+
+// The stages in reverse order, on small tables independent ones in one launch
+// (12 launches where one per stage takes 32; boxes whose pairs share a buffer
+// go pair by pair).
 void launch_all_adj(const EbAdjEnt *tab, const EbAdjEnt *htab, int n, const HydroConst &hc,
                     const double *dtp, hipStream_t st, Prof *prof, const CutCell *cells,
                     int ncells) {
