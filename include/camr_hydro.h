@@ -118,6 +118,8 @@ int camr_hydro_srctoprim(const camr_box *qbx, const camr_array4 *q,
  * Same contract: q, qaux, srcq cover grow(bx,4);
  * uin covers grow(bx,1); dsdt is ACCUMULATED (+=) on bx; flx[d] covers the
  * d-faces of bx and is overwritten with extensive (area-weighted) fluxes.
+ * (On the fused route below flux arrays may share memory, where the caller
+ * wants dsdt alone; the shared elements then hold any of their fluxes.)
  * area[d].p / vol->p may be NULL for a uniform Cartesian grid (then
  * area = product of the two other dx, vol = dx*dy*dz as geom.GetFaceArea /
  * GetVolume give); srcq->p may be NULL for identically +0 sources.
