@@ -3345,16 +3345,31 @@ int camr_version(void) { return 100; }
 } // extern "C"
 
 namespace {
+// Allows the calling thread's allocations while another thread captures a
+// stream (they touch no stream; in the default mode the runtime would refuse
+// them and void that capture).
+class RelaxedCapture {
+  public:
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+    RelaxedCapture(const RelaxedCapture &) = delete;
+    RelaxedCapture &operator=(const RelaxedCapture &) = delete;
+
+  private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
 // A few words of device memory and their pinned host mirror, for the
 // synchronous per-box calls that return a device result.  Taken for one
 // call (so calls of several threads and streams never share them) and put
 // back after it; up to kKeep sets per device are kept for later calls, more
 // are freed.  Bytes 0..31 hold anything, the status word at byte 32 is zero
-// in a kept set.
+// in a kept set.  All of it runs on the call's own stream: the null stream
+// would wait for the other streams, and void a capture among them.
 class CallWords {
   public:
     static constexpr size_t kBytes = 64, kStatus = 32;
-    CallWords() {
+    explicit CallWords(hipStream_t st) : st_(st) {
         if (hipGetDevice(&dev_) != hipSuccess) return;
         if (dev_ < kDevices) {
             std::lock_guard<std::mutex> g(mu());
@@ -3364,12 +3379,15 @@ class CallWords {
                 return;
             }
         }
+        RelaxedCapture relaxed;
         if (hipMalloc(&s_.dev, kBytes) != hipSuccess) { s_.dev = nullptr; return; }
         if (hipHostMalloc(&s_.host, kBytes) != hipSuccess || !zero_status()) drop();
     }
     // after the call's work has ended: the words may be kept, their status
     // word being `status`
-    void finished(int status) { keep_ = status == 0 || zero_status(); }
+    void finished(int status) {
+        keep_ = status == 0 || (zero_status() && hipStreamSynchronize(st_) == hipSuccess);
+    }
     ~CallWords() {
         if (!s_.dev) return;
         if (keep_ && dev_ < kDevices) {
@@ -3380,6 +3398,7 @@ class CallWords {
                 return;
             }
         }
+        RelaxedCapture relaxed;
         drop();  // hipFree waits for what an early return left running
     }
     CallWords(const CallWords &) = delete;
@@ -3407,14 +3426,16 @@ class CallWords {
         return k[dev];
     }
     bool zero_status() {
-        return hipMemset(s_.dev, 0, kBytes) == hipSuccess &&
-               hipStreamSynchronize(nullptr) == hipSuccess;
+        hipLaunchKernelGGL(k_fill_bytes, dim3(1), dim3(64), 0, st_, (uint8_t *)s_.dev,
+                           (int64_t)kBytes);
+        return hipGetLastError() == hipSuccess;
     }
     void drop() {
         if (s_.dev) (void)hipFree(s_.dev);
         if (s_.host) (void)hipHostFree(s_.host);
         s_ = Set{nullptr, nullptr};
     }
+    hipStream_t st_;
     int dev_ = 0;
     bool keep_ = false;
     Set s_{nullptr, nullptr};
@@ -3432,7 +3453,7 @@ int camr_hydro_ctoprim(const camr_box *qbx, const camr_array4 *u, const camr_arr
         return CAMR_ERR_SHAPE;
     }
     hipStream_t s = (hipStream_t)stream;
-    CallWords w;
+    CallWords w(s);
     if (!w.ok()) { set_error("camr_hydro_ctoprim: status word"); return CAMR_ERR_ALLOC; }
     launch_on(k_ctoprim, B, s, view(*u), view(*q), view(*qaux), make_const(*p), w.status());
     CAMR_HIP(hipMemcpyAsync(w.host(), w.status(), sizeof(int), hipMemcpyDeviceToHost, s));
@@ -3724,7 +3745,7 @@ int camr_estdt_hydro(const camr_box *bx, const camr_array4 *u, const double dx[3
     if (!covers(*u, B, NVAR)) { set_error("u must cover bx"); return CAMR_ERR_SHAPE; }
     hipStream_t s = (hipStream_t)stream;
     struct Result { unsigned long long m; int st; int pad; } h = {0x7fefffffffffffffULL, 0, 0};
-    CallWords w;
+    CallWords w(s);
     if (!w.ok()) { set_error("camr_estdt_hydro: result words"); return CAMR_ERR_ALLOC; }
     char *buf = w.dev();
     *(Result *)w.host() = h;
