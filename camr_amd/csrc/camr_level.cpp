@@ -3968,6 +3968,7 @@ int camr_level_set_zmarch(camr_level *L, const int32_t planes[CAMR_NSTAGE]) {
     int rc = L->impl.get_tuning(&t);
     if (rc) return rc;
     for (int k = 0; k < ST_COUNT; ++k) t.zm[k] = planes[k];
+    t.zm_set = 1;
     return L->impl.set_tuning(t);
 }
 int camr_level_set_ctu(camr_level *L, int32_t on, int32_t planes) {

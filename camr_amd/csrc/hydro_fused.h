@@ -440,6 +440,9 @@ struct Tuning {
     // z-march planes per thread (0: one point per thread); only the z-face
     // transverse stages (ST_T1 + 2, ST_T2 + 2) have marching kernels
     int zm[ST_COUNT];
+    // 1: zm was asked for by the caller (planes > 0 then keep the stage's
+    // directions in launches of their own, see merge_faces)
+    int zm_set;
     // 1: the transverse stages run as the LDS-staged CTU face kernels
     // (k_ctu_x/y/z, the transdo fluxes never stored); 0: the staged
     // k_trans1 / k_trans2 launches

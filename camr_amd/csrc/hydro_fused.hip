@@ -933,7 +933,7 @@ k_trans2(Batch B, HydroConst hc, const double *dtp) {
 }
 
 // All three directions in one launch, for levels whose launches are short
-// (see kMergeBlocks).
+// (see kMergeThreads).
 template <int D>
 __device__ __forceinline__ void trans1_any(const Batch &B, int w, int nw, const HydroConst &hc,
                                            const double *dtp) {
@@ -1534,19 +1534,19 @@ k_update_c(Batch B, HydroConst hc, const double *dtp, int *flags) {
 } // namespace
 
 // --------------------------------------------------------------- engine
-// block prefix rows: the stage kinds as tuned, the same without z-march
-// (LaunchCfg linear), then the CTU face kernels and the trace + first-flux
-// kernels of the three directions
-
 // The transverse stages' three directions run as one launch up to this many
-// blocks.  Measured, one launch against three per stage (us per step or
+// threads.  Measured, one launch against three per stage (us per step or
 // call): 256x4x4 PLM 121 against 162, 32^3 level 152 / 176, 64^3 455 / 493,
 // 97x83x61 995 / 1018, 42 refined boxes of 8..32 5250 / 5408 (four steps),
-// 128^3 2861 / 2885, 160^3 (5.0e4 blocks) 5356 / 5357, 256^3 (2.0e5)
+// 128^3 2861 / 2885, 160^3 (1.28e7 threads) 5356 / 5357, 256^3 (5.1e7)
 // 21214 / 20786: launches and last waves cost the small ones, while a large
 // one gains more from the z-marching kernels and from registers sized for
 // one direction.
-constexpr int64_t kMergeBlocks = 49152;
+constexpr int64_t kMergeThreads = 49152 * (int64_t)kBlock;
+
+// block prefix rows: the stage kinds as tuned, the same without z-march
+// (LaunchCfg linear), then the CTU face kernels and the trace + first-flux
+// kernels of the three directions
 constexpr int kCtuRow0 = 2 * ST_COUNT, kFace1Row0 = kCtuRow0 + 3, kBlkRows = kFace1Row0 + 3;
 
 Tuning default_tuning() {
@@ -1559,6 +1559,7 @@ Tuning default_tuning() {
         t.zm[k] = 0;
     }
     t.zm[ST_T1 + 2] = t.zm[ST_T2 + 2] = 2;
+    t.zm_set = 0;
     t.order = 0;
     t.ctu = 0;
     t.ctu_planes = 8;
@@ -1763,15 +1764,17 @@ LaunchCfg FusedEngine::cfg(int kind, int b, int parity, bool linear) const {
 }
 
 // The three directions of a transverse stage as one launch: for linear and
-// tiled blocks of one size, up to kMergeBlocks blocks.
+// tiled blocks of one size, up to kMergeThreads threads, unless the caller set
+// a z-march (the merged kernels have none).
 bool FusedEngine::merge_faces(int kind, int b, int parity, LaunchCfg c[3]) const {
+    if (tune_.zm_set && tune_.zm[kind + 2] > 0) return false;
     int64_t n = 0;
     for (int d = 0; d < 3; ++d) {
         c[d] = cfg(kind + d, b, parity, true);
         if (c[d].block != c[0].block) return false;
-        n += c[d].grid;
+        n += (int64_t)c[d].grid * c[d].block;
     }
-    return n <= kMergeBlocks;
+    return n <= kMergeThreads;
 }
 
 LaunchCfg FusedEngine::cfg_face1(int d, int b, int parity) const {

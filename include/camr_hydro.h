@@ -426,7 +426,10 @@ int camr_level_get_xcd(camr_level *L, int32_t chunk[CAMR_NSTAGE]);
  * stages (transdo pairs and transdd, stage ranges 7 and 11) with linear
  * blocks take it; camr_level_set_tiles clears it for tiled stages.  Results
  * do not depend on it.  camr_level_set_tuning resets it to 2 for those two
- * stages and 0 elsewhere.  No reference counterpart: set by the autotuner. */
+ * stages and 0 elsewhere.  Small levels run the three directions of a
+ * transverse stage in one launch, without a march, as long as the planes are
+ * that default or 0; P > 0 set here is taken at any size.  No reference
+ * counterpart. */
 int camr_level_set_zmarch(camr_level *L, const int32_t planes[CAMR_NSTAGE]);
 int camr_level_get_zmarch(camr_level *L, int32_t planes[CAMR_NSTAGE]);
 /* LDS-staged CTU face kernels: on = 1 runs the transverse stages of each

@@ -1,7 +1,8 @@
 """The transverse stages as one launch per direction and as one launch of
-all three (levels up to kMergeBlocks blocks): both against the oracle, bit
+all three (levels up to kMergeThreads threads): both against the oracle, bit
 for bit.  Block sizes that differ between the directions (or between the
-flattening and the nodal divergence) keep the launches apart at any size."""
+flattening and the nodal divergence) keep the launches apart at any size, and
+so does a z-march set by the caller."""
 import numpy as np
 import pytest
 
