@@ -41,6 +41,7 @@ class MolEngine {
     int source(const HydroConst &hc, hipStream_t st, int *status, Prof *prof) const;
 
   private:
+    void release();
     std::vector<MolBox> host_;
     std::vector<int> blk_host_;  // block prefixes: cells, nodes, x-y tiles, x-z tiles
     MolBox *tab_ = nullptr;

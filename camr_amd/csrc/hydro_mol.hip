@@ -269,10 +269,15 @@ k_mol_z(const MolBox *tab, const int *blk, int nbox, HydroConst hc) {
 
 bool MolEngine::fits(const Box &bx) { return canon_fits(bx); }
 
-MolEngine::~MolEngine() {
+MolEngine::~MolEngine() { release(); }
+
+void MolEngine::release() {
     if (tab_) (void)hipFree(tab_);
     if (blk_) (void)hipFree(blk_);
     if (buf_) (void)hipFree(buf_);
+    tab_ = nullptr;
+    blk_ = nullptr;
+    buf_ = nullptr;
 }
 
 int MolEngine::setup(const std::vector<Box> &boxes, const std::vector<Arr> &sb,
@@ -281,16 +286,17 @@ int MolEngine::setup(const std::vector<Box> &boxes, const std::vector<Arr> &sb,
     host_.resize(n);
     size_t total = 0;
     for (const Box &b : boxes) total += ((size_t)(NQC + 1) * canon_box(b).npts() + 31) & ~size_t(31);
-    // where the primitives of all boxes at once are much of what is free, the
-    // level stays with one box's scratch per stream
+    // where the primitives of all boxes at once are much of what is free, or
+    // are not to be had, the level stays with one box's scratch per stream
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || total * sizeof(double) > free_b / 4)
         return CAMR_OK;
     if (hipMalloc(&buf_, total * sizeof(double)) != hipSuccess ||
         hipMalloc(&blk_, (size_t)4 * (n + 1) * sizeof(int)) != hipSuccess ||
         hipMalloc(&tab_, std::max(n, 1) * sizeof(MolBox)) != hipSuccess) {
-        set_error("method of lines: allocation of %zu bytes failed", total * sizeof(double));
-        return CAMR_ERR_ALLOC;
+        release();
+        (void)hipGetLastError();  // not a later launch's
+        return CAMR_OK;
     }
     blk_host_.assign((size_t)4 * (n + 1), 0);
     double *p = buf_;
