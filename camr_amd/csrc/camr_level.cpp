@@ -263,7 +263,11 @@ class HydroLevel {
     // the cut-cell boxes' / the adjoint's scratch has a buffer per transverse
     // pair (EbBox::keep)
     bool eb_keep_ = false, eadj_keep_ = false;
+    bool eb_lean_ = false;  // memory ran short: no such buffers from now on
     bool eb_keep(const std::vector<Box> &bs) const;
+    int place_cut_boxes();
+    bool drop_pair_buffers();
+    int adjoint_buffers(int nck, int every);
     std::vector<Box> vbox_;
     int nmerged_ = 0;
     int *vg_ids_ = nullptr;
@@ -284,8 +288,7 @@ class HydroLevel {
     std::vector<EbGeom> ebg_;
     std::vector<double *> ebbuf_;
     // the cut-cell boxes (kind 1) as one table of the batched EB path, each
-    // with its own q / qaux / srcq, fluxes and scratch in cut_buf_ (freed
-    // with ebbuf_)
+    // with its own q / qaux / srcq, fluxes and scratch in cut_buf_
     std::vector<int> cut_ids_;
     std::vector<size_t> cut_off_;
     std::vector<EbBox> cut_htab_;
@@ -700,6 +703,10 @@ void HydroLevel::release() {
     nws_ = 0;
     for (auto p : ebbuf_) fr(p);
     ebbuf_.clear();
+    fr(cut_buf_);
+    fr(eadj_fbuf_);
+    fr(eadj_abuf_);
+    cut_buf_ = eadj_fbuf_ = eadj_abuf_ = nullptr;
     if (h_dtmin_) (void)hipHostFree(h_dtmin_);
     tab_old_ = tab_sb_ = tab_src_ = nullptr;
     owner_ = status_ = nullptr;
@@ -995,29 +1002,17 @@ int HydroLevel::set_eb(const int32_t *flags, const int32_t flo[3], const int32_t
     cut_cells_ = nullptr;  // (an earlier list is freed with ebbuf_)
     ncut_cells_ = 0;
     cut_cells_h_.clear();
-    size_t tot = 0;
-    auto r32 = [](size_t n) { return (n + 31) / 32 * 32; };
-    std::vector<Box> cut;
     for (int b = 0; b < nb; ++b)
-        if (kind_[b] == 1) cut.push_back(box_[b]);
-    eb_keep_ = eb_keep(cut);
-    for (int b = 0; b < nb; ++b) {
-        if (kind_[b] != 1) continue;
-        const Box B = box_[b], G = grow(B, ng_);
-        cut_ids_.push_back(b);
-        cut_off_.push_back(tot);
-        tot += r32((size_t)(2 * QVAR + NQAUX) * G.npts());
-        for (int d = 0; d < 3; ++d) tot += r32((size_t)NVAR * nodes(B, d).npts());
-        tot += r32(umdrv_eb_scratch_doubles(B, G, eb_keep_));
-    }
+        if (kind_[b] == 1) cut_ids_.push_back(b);
     if (!cut_ids_.empty()) {
-        CAMR_HIP(hipMalloc(&cut_buf_, tot * sizeof(double)));
-        ebbuf_.push_back(cut_buf_);
         CAMR_HIP(hipMalloc(&cut_tab_, cut_ids_.size() * sizeof(EbBox)));
         ebbuf_.push_back(reinterpret_cast<double *>(cut_tab_));
-        cut_htab_.assign(cut_ids_.size(), EbBox{});
-        for (size_t c = 0; c < cut_ids_.size(); ++c)
-            if ((rc = cut_entry((int)c))) return rc;
+        std::vector<Box> cut;
+        for (int b : cut_ids_) cut.push_back(box_[b]);
+        eb_keep_ = eb_keep(cut);
+        rc = place_cut_boxes();
+        if (rc && drop_pair_buffers()) rc = CAMR_OK;
+        if (rc) return rc;
         // the cut cells, for the cut-cell divergence (the cells where
         // b_eb_div<true> acts)
         std::vector<CutCell> cells;
@@ -1337,8 +1332,50 @@ bool HydroLevel::eb_keep(const std::vector<Box> &bs) const {
         const Box G = grow(B, ng_);
         more += umdrv_eb_scratch_doubles(B, G, true) - umdrv_eb_scratch_doubles(B, G, false);
     }
-    return eb_merge_ && hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
+    return eb_merge_ && !eb_lean_ && hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
            more * sizeof(double) <= free_b / 8;
+}
+
+// The cut-cell boxes' arrays (eb_keep_: with a buffer per transverse pair) and
+// their table entries.
+int HydroLevel::place_cut_boxes() {
+    auto r32 = [](size_t n) { return (n + 31) / 32 * 32; };
+    size_t tot = 0;
+    cut_off_.clear();
+    for (int b : cut_ids_) {
+        const Box B = box_[b], G = grow(B, ng_);
+        cut_off_.push_back(tot);
+        tot += r32((size_t)(2 * QVAR + NQAUX) * G.npts());
+        for (int d = 0; d < 3; ++d) tot += r32((size_t)NVAR * nodes(B, d).npts());
+        tot += r32(umdrv_eb_scratch_doubles(B, G, eb_keep_));
+    }
+    CAMR_HIP(hipMalloc(&cut_buf_, tot * sizeof(double)));
+    cut_htab_.assign(cut_ids_.size(), EbBox{});
+    for (size_t c = 0; c < cut_ids_.size(); ++c) {
+        const int rc = cut_entry((int)c);
+        if (rc) return rc;
+    }
+    return CAMR_OK;
+}
+
+// After an allocation of an EB level has failed: gives up the buffers per
+// transverse pair (the stages then run pair by pair).  True if that freed
+// memory, or lets the allocation that failed be smaller: it is worth trying
+// again.
+bool HydroLevel::drop_pair_buffers() {
+    if (!eb_keep_ && !eadj_keep_) return false;
+    (void)hipGetLastError();  // the failure's
+    if (hipStreamSynchronize(stream_) != hipSuccess) return false;
+    release_graphs();
+    eb_lean_ = true;
+    eadj_keep_ = false;
+    if (eadj_abuf_) (void)hipFree(eadj_abuf_);
+    eadj_abuf_ = nullptr;
+    if (!eb_keep_) return true;
+    eb_keep_ = false;
+    if (cut_buf_) (void)hipFree(cut_buf_);
+    cut_buf_ = nullptr;
+    return place_cut_boxes() == CAMR_OK;
 }
 
 // Table entry c of the cut-cell batch: box cut_ids_[c] with its arrays in
@@ -2105,6 +2142,13 @@ int HydroLevel::load_state(const double *src) {
 }
 
 int HydroLevel::adjoint_alloc(int nck, int every) {
+    int rc = adjoint_buffers(nck, every);
+    if (rc && drop_pair_buffers()) rc = adjoint_buffers(nck, every);
+    return rc;
+}
+
+// What adjoint_alloc allocates and does not have yet.
+int HydroLevel::adjoint_buffers(int nck, int every) {
     int rc = ebflags_ ? eb_adjoint_setup() : engine_.enable_adjoint();
     if (rc) return rc;
     state_doubles_ = 0;
@@ -2117,19 +2161,20 @@ int HydroLevel::adjoint_alloc(int nck, int every) {
         CAMR_HIP(hipMalloc(&state_off_, off.size() * sizeof(int64_t)));
         CAMR_HIP(hipMemcpy(state_off_, off.data(), off.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     }
-    if (abar_[0].empty()) {
-        for (int q = 0; q < 2; ++q) {
-            std::vector<DevFab> t(box_.size());
-            for (size_t b = 0; b < box_.size(); ++b) {
-                double *p = nullptr;
-                CAMR_HIP(hipMalloc(&p, NVAR * box_[b].npts() * sizeof(double)));
-                abar_[q].push_back(p);
-                t[b].a = dense(p, box_[b]);
-                t[b].b = box_[b];
-            }
-            CAMR_HIP(hipMalloc(&tab_abar_[q], box_.size() * sizeof(DevFab)));
-            CAMR_HIP(hipMemcpy(tab_abar_[q], t.data(), box_.size() * sizeof(DevFab), hipMemcpyHostToDevice));
+    for (int q = 0; q < 2; ++q) {
+        while (abar_[q].size() < box_.size()) {
+            double *p = nullptr;
+            CAMR_HIP(hipMalloc(&p, NVAR * box_[abar_[q].size()].npts() * sizeof(double)));
+            abar_[q].push_back(p);
         }
+        if (tab_abar_[q]) continue;
+        std::vector<DevFab> t(box_.size());
+        for (size_t b = 0; b < box_.size(); ++b) {
+            t[b].a = dense(abar_[q][b], box_[b]);
+            t[b].b = box_[b];
+        }
+        CAMR_HIP(hipMalloc(&tab_abar_[q], box_.size() * sizeof(DevFab)));
+        CAMR_HIP(hipMemcpy(tab_abar_[q], t.data(), box_.size() * sizeof(DevFab), hipMemcpyHostToDevice));
     }
     while ((int)ckpt_.size() < nck) {
         double *p = nullptr;
@@ -2248,6 +2293,7 @@ int HydroLevel::adjoint_flags() {
 // box tables (rebuilt on every call, so that geometry set later is seen).
 int HydroLevel::eb_adjoint_setup() {
     const int nb = (int)box_.size();
+    auto r32 = [](size_t n) { return (n + 31) / 32 * 32; };
     if (!eadj_fbuf_) {
         // regular geometry for the all-regular boxes: constant rows indexed
         // by i only (zero j / k / component strides)
@@ -2284,33 +2330,13 @@ int HydroLevel::eb_adjoint_setup() {
         for (int b = 0; b < nb; ++b)
             if (kind_[b] != 2 && (vof_.empty() || vof_[b] < 0)) eadj_ids_.push_back(b);
         for (size_t v = 0; v < vbox_.size(); ++v) eadj_ids_.push_back(-1 - (int)v);
-        auto r32 = [](size_t n) { return (n + 31) / 32 * 32; };
-        size_t fn = 0, an = 0;
         std::vector<Box> run;
         for (int id : eadj_ids_) run.push_back(id >= 0 ? box_[id] : vbox_[-1 - id]);
         eadj_keep_ = eb_keep(run);
-        for (int id : eadj_ids_) {
-            const Box B = id >= 0 ? box_[id] : vbox_[-1 - id], G = grow(B, ng_);
-            fn += r32((size_t)(QVAR + NQAUX) * G.npts());
-            for (int d = 0; d < 3; ++d) fn += r32((size_t)NVAR * nodes(B, d).npts());
-            fn += r32(umdrv_eb_scratch_doubles(B, G, true));
-            an += r32((size_t)(QVAR + NQAUX) * G.npts());
-            an += r32(umdrv_eb_scratch_doubles(B, G, eadj_keep_));
-        }
-        for (int b = 0; b < nb; ++b)
-            an += r32((size_t)NVAR * box_[b].npts()) + r32((size_t)NVAR * grow(box_[b], ng_).npts());
-        for (const Box &V : vbox_)
-            an += r32((size_t)NVAR * V.npts()) + r32((size_t)NVAR * grow(V, ng_).npts());
         if (!vbox_.empty()) {
             CAMR_HIP(hipMalloc(&vga_dev_, vbox_.size() * sizeof(VGather)));
             ebbuf_.push_back(reinterpret_cast<double *>(vga_dev_));
         }
-        CAMR_HIP(hipMalloc(&eadj_fbuf_, fn * sizeof(double)));
-        ebbuf_.push_back(eadj_fbuf_);
-        CAMR_HIP(hipMalloc(&eadj_abuf_, an * sizeof(double)));
-        ebbuf_.push_back(eadj_abuf_);
-        eadj_an_ = an;
-
         const size_t n = eadj_ids_.size();
         CAMR_HIP(hipMalloc(&eadj_ftab_, std::max<size_t>(n, 1) * sizeof(EbBox)));
         ebbuf_.push_back(reinterpret_cast<double *>(eadj_ftab_));
@@ -2324,9 +2350,30 @@ int HydroLevel::eb_adjoint_setup() {
         ebbuf_.push_back(reinterpret_cast<double *>(geom_dev_));
         CAMR_HIP(hipMalloc(&kinds_dev_, nb * sizeof(int)));
         ebbuf_.push_back(reinterpret_cast<double *>(kinds_dev_));
+        size_t fn = 0;
+        for (const Box &B : run) {
+            const Box G = grow(B, ng_);
+            fn += r32((size_t)(QVAR + NQAUX) * G.npts());
+            for (int d = 0; d < 3; ++d) fn += r32((size_t)NVAR * nodes(B, d).npts());
+            fn += r32(umdrv_eb_scratch_doubles(B, G, true));
+        }
+        CAMR_HIP(hipMalloc(&eadj_fbuf_, fn * sizeof(double)));
+    }
+    if (!eadj_abuf_) {
+        size_t an = 0;
+        for (int id : eadj_ids_) {
+            const Box B = id >= 0 ? box_[id] : vbox_[-1 - id], G = grow(B, ng_);
+            an += r32((size_t)(QVAR + NQAUX) * G.npts());
+            an += r32(umdrv_eb_scratch_doubles(B, G, eadj_keep_));
+        }
+        for (int b = 0; b < nb; ++b)
+            an += r32((size_t)NVAR * box_[b].npts()) + r32((size_t)NVAR * grow(box_[b], ng_).npts());
+        for (const Box &V : vbox_)
+            an += r32((size_t)NVAR * V.npts()) + r32((size_t)NVAR * grow(V, ng_).npts());
+        CAMR_HIP(hipMalloc(&eadj_abuf_, an * sizeof(double)));
+        eadj_an_ = an;
     }
     // tables
-    auto r32 = [](size_t n) { return (n + 31) / 32 * 32; };
     double *fp = eadj_fbuf_, *ap = eadj_abuf_;
     std::vector<Arr> ubv(box_.size()), sbbv(box_.size());
     std::vector<EbGeom> geo(box_.size());

@@ -73,8 +73,72 @@ static void mol() {
            launches[1]);
 }
 
+// Cut-cell boxes: the buffers per transverse pair (forward and adjoint) are
+// given up where the level, its gradient or more checkpoints would not fit
+// with them; what pair by pair needs is enough, and less than that is refused.
+struct EbRun {
+    int made = 0, grad = 0, again = 0;  // return codes of the three
+    size_t peak = 0;
+};
+static EbRun eb(int merge, size_t cap) {
+    const int n = 16;
+    const std::vector<int32_t> boxes = {0, 0, 0, 15, 15, 7, 0, 0, 8, 15, 15, 15};
+    camr_level_desc d = desc(n, boxes);
+    d.hp.ppm_type = 0;
+    d.engine = 1;
+    d.fixed_dt = 1e-3;
+    fake::cap = cap;
+    fake::peak = 0;
+    fake::last = hipSuccess;
+    EbRun r;
+    camr_level *L = nullptr;
+    r.made = camr_level_create(&d, &L);
+    const int32_t flo[3] = {-7, -7, -7}, fhi[3] = {n + 6, n + 6, n + 6};
+    const int m = n + 14;
+    std::vector<int32_t> flags((size_t)m * m * m, (1 << 27) - 1);
+    for (int k : {4, 12})  // a cut cell in each box
+        flags[(8 + 7) + (8 + 7) * m + (size_t)(k + 7) * m * m] |= 1 << 27;
+    if (!r.made) r.made = camr_level_set_eb_merge(L, merge);
+    if (!r.made) r.made = camr_level_set_eb(L, flags.data(), flo, fhi);
+    std::vector<double> one((size_t)(n + 15) * (n + 15) * 23, 1.0), off(2 * one.size(), 0.0);
+    for (int b = 0; b < 2 && !r.made; ++b)
+        r.made = camr_level_set_box_eb(L, b, one.data(), one.data(), one.data(), one.data(),
+                                       off.data(), off.data(), off.data());
+    const std::vector<double> dts(6, 1e-3);
+    auto gradient = [&](int steps, int every) {
+        int rc = camr_level_adjoint_forward(L, steps, dts.data(), every);
+        return rc ? rc : camr_level_adjoint_backward(L);
+    };
+    if (!r.made && !(r.grad = gradient(1, 1))) r.again = gradient(6, 2);
+    if (!r.made && !r.grad && !r.again) CHECK(fake::last == hipSuccess, "error left");
+    if (L) camr_level_destroy(L);
+    CHECK(fake::used == 0, "%zu bytes left", fake::used);
+    r.peak = fake::peak;
+    fake::cap = size_t(1) << 40;
+    return r;
+}
+static void eb_levels() {
+    const EbRun lean = eb(0, fake::cap), full = eb(1, fake::cap);
+    CHECK(!lean.made && !lean.grad && !lean.again, "%d %d %d", lean.made, lean.grad, lean.again);
+    CHECK(!full.made && !full.grad && !full.again, "%d %d %d", full.made, full.grad, full.again);
+    CHECK(full.peak > lean.peak, "%zu, %zu bytes", full.peak, lean.peak);
+    for (int s = 0; s <= 40; ++s) {
+        const size_t cap = lean.peak + (full.peak - lean.peak) * s / 40;
+        const EbRun r = eb(1, cap);
+        CHECK(!r.made && !r.grad && !r.again, "%zu of %zu bytes: %d %d %d", cap, full.peak, r.made,
+              r.grad, r.again);
+    }
+    for (int merge = 0; merge < 2; ++merge)
+        for (int s = 1; s < 40; ++s) {
+            const EbRun r = eb(merge, lean.peak * s / 40);
+            CHECK(r.made || r.grad || r.again, "%d of 40 accepted", s);
+        }
+    printf("cut cells: %zu bytes pair by pair, %zu with a buffer per pair\n", lean.peak, full.peak);
+}
+
 int main() {
     mol();
+    eb_levels();
     printf(bad ? "%d FAILED\n" : "LEVEL MEMORY OK\n", bad);
     return bad != 0;
 }
