@@ -57,7 +57,7 @@ STAGES = {
     "trace_riemann": (2, 3, 4),  # only the XCD chunk: the stage has its own blocks
     "transverse_1": (5, 6, 7),
     "transverse_2": (9, 10, 11),
-    "consup": (12,), "clean_estdt": (12,), "consup_clean_estdt": (12,),
+    "consup": (12,), "consup_clean_estdt": (12,),
 }
 # groups of stage ranges that must share a block size (one profiler name)
 GROUPS = [(0,), (1, 8), (2, 3, 4), (5, 6, 7), (9, 10, 11), (12,)]

@@ -422,7 +422,6 @@ struct LaunchCfg {
     int block;
 };
 void launch_fill_fused(const LaunchCfg &c, const FillArgs &a, hipStream_t st, int *status);
-void launch_post_fused(const LaunchCfg &c, const PostArgs &a, hipStream_t st, int *status);
 // S_new from the fill's Sborder copy (new_values), the update of k_update_c
 // and the post pass in one kernel (S_new only written).
 void launch_update_post_fused(const LaunchCfg &c, const HydroConst &hc, const double *dtp,
@@ -473,17 +472,17 @@ class FusedEngine {
     // and energy checks into *status.  have_prim: fill() already wrote the
     // primitives, the Sborder copy and the primitive sources; else they come
     // from sb_tab (and the sources from src_tab).  has_src: SRC_*.
-    // With `post`, the update and the post pass (post()) run as one kernel;
-    // with `no_update` the final update is left out (the fluxes are ready in
-    // the scratch, S_new is not touched).
+    // With `post`, S_new is formed from fill()'s Sborder copy, updated and
+    // passed through the post pass in one kernel; without, the update is added
+    // to an S_new that holds Sborder + dt * old source (never after fill());
+    // with `no_update` it is left out (the fluxes are ready in the scratch,
+    // S_new is not touched).
     int hydro(int b, int parity, bool have_prim, const DevFab *sb_tab, const DevFab *src_tab,
               int has_src, const HydroConst &hc, const double *dtp, hipStream_t st,
               int *status, Prof *prof, const PostArgs *post = nullptr,
               bool no_update = false);
-    // ghost fill + clean + primitives + S_new = Sborder + dt * old source
+    // ghost fill + clean + primitives (+ their sources)
     int fill(int b, int parity, const FillArgs &a, hipStream_t st, int *status, Prof *prof);
-    // clean_state passes after the update + next dt estimate
-    int post(int b, int parity, const PostArgs &a, hipStream_t st, int *status, Prof *prof);
     // after hydro(..., no_update = true): hydro_pdivu + hydro_update of
     // every box into dsdt_tab[id] (overwritten, the staged path's zero fill
     // and += order), for callers that apply dS/dt themselves

@@ -1926,14 +1926,6 @@ int FusedEngine::dsdt(int b, int parity, const DevFab *dsdt_tab, const HydroCons
     return hipGetLastError() == hipSuccess ? CAMR_OK : CAMR_ERR_HIP;
 }
 
-int FusedEngine::post(int b, int parity, const PostArgs &a, hipStream_t st, int *status,
-                      Prof *prof) {
-    const LaunchCfg c = cfg(ST_VALID, b, parity);
-    Region reg(prof, "clean_estdt", st);
-    launch_post_fused(c, a, st, status);
-    return hipGetLastError() == hipSuccess ? CAMR_OK : CAMR_ERR_HIP;
-}
-
 // ------------------------------------------------------- one-box route
 namespace {
 constexpr size_t kOneBoxHeader = 64;  // doubles ahead of the canonical arrays (512 bytes)

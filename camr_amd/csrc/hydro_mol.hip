@@ -14,7 +14,7 @@
 // waits half its time).  All three directions in one launch, marching in z,
 // need 256 VGPRs: 577 us at two waves per SIMD.
 // The arithmetic per face and cell is theirs (mol_slopes, mol_face_state,
-// face_flux, adjust_face_vals, hydro_update's order), hence the same bits.
+// face_flux, adjust_face_jump, hydro_update's order), hence the same bits.
 #include "hydro_mol.h"
 #include "hydro_fused.h"
 #include "hydro_kernels.h"

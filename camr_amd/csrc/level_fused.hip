@@ -136,27 +136,7 @@ __device__ __forceinline__ double post_values(const BoxEnt &E, int i, int j, int
     return dtv;
 }
 
-__global__ void __launch_bounds__(kBlock)
-k_post_fused(Batch B, PostArgs a, int *status) {
-    if (B.halt && *B.halt) return;  // uniform: the whole block leaves
-    int lblk;
-    const BoxEnt &E = B.tab[batch_box(B, lblk)];
-    int i, j, k;
-    double dtv = 1.7976931348623157e308;
-    // every thread reaches the block reduction below
-    if (batch_point(B, E.bx, lblk, i, j, k)) {
-        const Arr snew = E.snew;
-        double v[NVAR];
-#pragma unroll
-        for (int n = 0; n < NVAR; ++n) v[n] = snew(i, j, k, n);
-        dtv = post_values(E, i, j, k, a, v);
-#pragma unroll
-        for (int n = 0; n < NVAR; ++n) snew(i, j, k, n) = v[n];
-    }
-    block_min_commit(dtv, a.dtmin, status);
-}
-
-// new_values, k_update_c and k_post_fused, with S_new kept in registers in
+// new_values, k_update_c and post_values, with S_new kept in registers in
 // between (the same arithmetic: S_new is rounded once by each either way).
 // Written by the fill and read back here it cost 1.3 GB at 256^3: fill 1.33 ->
 // 0.95 ms, this kernel 1.70 -> 1.65 ms.
@@ -172,6 +152,7 @@ k_update_post(Batch B, HydroConst hc, const double *dtp, PostArgs a, int *status
     const BoxEnt &E = B.tab[batch_box(B, lblk)];
     int i, j, k;
     double dtv = 1.7976931348623157e308;
+    // every thread reaches the block reduction below
     if (batch_point(B, E.bx, lblk, i, j, k)) {
         const Arr snew = E.snew;
         const Arr sold = E.sold;
@@ -198,11 +179,6 @@ k_update_post(Batch B, HydroConst hc, const double *dtp, PostArgs a, int *status
 void launch_fill_fused(const LaunchCfg &c, const FillArgs &a, hipStream_t st, int *status) {
     if (c.grid == 0) return;
     hipLaunchKernelGGL(k_fill_fused, dim3(c.grid), dim3(c.block), 0, st, c.B, a, status);
-}
-
-void launch_post_fused(const LaunchCfg &c, const PostArgs &a, hipStream_t st, int *status) {
-    if (c.grid == 0) return;
-    hipLaunchKernelGGL(k_post_fused, dim3(c.grid), dim3(c.block), 0, st, c.B, a, status);
 }
 
 void launch_update_post_fused(const LaunchCfg &c, const HydroConst &hc, const double *dtp,
