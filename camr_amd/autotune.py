@@ -25,9 +25,9 @@ stage, since a stage's cost depends only on its own launch shape); the
 fastest candidate per stage range is kept (the three directions of a face
 stage share one profiler name, so they share one candidate).  The combined
 choice is then checked against the default on whole steps and kept only if
-faster.  Results are cached in a JSON file keyed by the device name and the
-histogram of box sizes, so a level with the same box population reuses
-them without timing anything.
+faster.  Results are cached in a JSON file keyed by the device name, the
+launch structure (LAUNCHES) and the histogram of box sizes, so a level with
+the same box population reuses them without timing anything.
 """
 from __future__ import annotations
 
@@ -61,6 +61,19 @@ STAGES = {
 }
 # groups of stage ranges that must share a block size (one profiler name)
 GROUPS = [(0,), (1, 8), (2, 3, 4), (5, 6, 7), (9, 10, 11), (12,)]
+# Version of what a launch holds.  A cached choice was timed with the launches
+# of its time: block sizes picked for stages that now share a launch would
+# keep them apart.  It goes up when stages are merged or split, or a stage
+# takes other settings.
+LAUNCHES = 2
+
+
+def candidates(grp):
+    """The candidates that make a difference for a group of stage ranges: the
+    first-flux faces have blocks of their own and take only the XCD chunk."""
+    if grp == (2, 3, 4):
+        return [c for c in CANDIDATES if c[:2] == (256, LINEAR)]
+    return list(CANDIDATES)
 
 
 def cache_path() -> str:
@@ -70,10 +83,10 @@ def cache_path() -> str:
 
 
 def key_of(level, device: str) -> str:
-    """Device + ppm_type + histogram of box shapes."""
+    """Device + launch structure + ppm_type + histogram of box shapes."""
     shapes = sorted(tuple(b[3 + d] - b[d] + 1 for d in range(3)) for b in level.prob.boxes)
     h = hashlib.sha1(repr(shapes).encode()).hexdigest()[:16]
-    return f"{device}|ppm{level.prob.value('ppm_type')}|{len(shapes)}boxes|{h}"
+    return f"{device}|launches{LAUNCHES}|ppm{level.prob.value('ppm_type')}|{len(shapes)}boxes|{h}"
 
 
 def _device_name() -> str:
@@ -131,7 +144,8 @@ def report_markdown(table, results, t_def) -> str:
         if order != 0:
             continue
         best = min(cost.values())
-        cells = [(f"**{cost[c]:.3f}**" if cost[c] == best else f"{cost[c]:.3f}") for c in CANDIDATES]
+        cells = ["" if c not in cost else f"**{cost[c]:.3f}**" if cost[c] == best
+                 else f"{cost[c]:.3f}" for c in CANDIDATES]
         out.append(f"| {','.join(map(str, grp))} | " + " | ".join(cells) + " |")
     out += ["", "| whole step | ms |", "|---|---:|", f"| defaults | {t_def * 1e3:.3f} |"]
     for t, blocks, order, tiles, xcd, ctu in results:
@@ -182,7 +196,7 @@ def tune(level, steps: int = 3, use_cache: bool = True, verbose: bool = False):
         xcd = [0] * _lib.NSTAGE
         for grp in GROUPS:
             names = [n for n, st in STAGES.items() if st == grp or set(st) & set(grp)]
-            cost = {c: sum(times[(order, c)].get(n, 0.0) for n in names) for c in CANDIDATES}
+            cost = {c: sum(times[(order, c)].get(n, 0.0) for n in names) for c in candidates(grp)}
             table.append((order, grp, cost))
             pick = min(cost, key=cost.get)
             for g in grp:
