@@ -55,15 +55,15 @@ NS_MOL_READ, NF_MOL_WRITE = 23, 12
 # (profiles/hbm_traffic_fused_256cube_ppm.md, profiles/ctu_faces_256cube_ppm.md;
 # FETCH_SIZE scaled by 1.9692, WRITE_SIZE by 0.9961, the factors an
 # 8-byte-lane copy of 1 GiB reads back).  Reported only for that engine and size.
-MEASURED_TRAFFIC = {("fused", 256, "transverse_2"): 10447411888,
-                    ("fused", 256, "trace_riemann"): 18670000000,
+MEASURED_TRAFFIC = {("fused", 256, "transverse_2"): 10387821835,
+                    ("fused", 256, "trace_riemann"): 18848641598,
                     ("fused", 256, "transverse_ctu"): 28527364887}
 
 # Executed FP64 work of one PPM cell-update (ADD, MUL, TRANS = 1, FMA = 2 per
 # lane; FMAs only from the division / square-root expansions, contraction is
 # off), summed over the step's kernels from rocprofv3 SQ_INSTS_VALU_*_F64
 # counters at 256^3 (profiles/valu_fused_256cube_ppm.md).
-FP64_EXECUTED_PER_CELL_UPDATE = 10069
+FP64_EXECUTED_PER_CELL_UPDATE = 10202
 
 # Algorithmic FP64 operations of the reference's path per cell-update, by
 # stage (add/sub, mul, div, sqrt = 1 each; no FMA): the oracle run with an

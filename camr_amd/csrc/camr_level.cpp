@@ -332,7 +332,8 @@ class HydroLevel {
     double *ext_ = nullptr;     // exterior data (whole domain), when set
     double *cstage_ = nullptr;  // coarse values staged for exterior_from
     size_t cstage_n_ = 0;
-    // the domain cells that the boxes' ghost regions map to and no box owns (x, y, z triples; built on the first ghost fill)
+    // the domain cells that the boxes' ghost regions map to and no box owns
+    // (x, y, z triples; built on the first ghost fill)
     int *shell_cells_ = nullptr;
     int64_t shell_n_ = -1;
     // the coarse cells (grown coarse domain) their interpolation reads, for
@@ -571,8 +572,8 @@ void HydroLevel::drop_shell_cells() {
 
 // The lists are made on the device: marks, then the marked cells counted and
 // written.  (By a host loop over the grown boxes and the domain they were half
-// of the first pass of a 96^3 level with a refined block in it: 15.5 ms, now
-// 7.0.)  Their order is that of the atomics, so only the cells' grouping into
+// of the first pass of a 96^3 level with a refined block in it: 14.5 ms, now
+// 6.4.)  Their order is that of the atomics, so only the cells' grouping into
 // blocks varies.
 int HydroLevel::build_shell_cells(int ratio, const Box &cdom) {
     drop_shell_cells();

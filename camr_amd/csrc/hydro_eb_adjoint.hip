@@ -927,7 +927,9 @@ constexpr const char *adj_name(int s) {
 
 // AS_DIVCUT / AS_RSRC over a list of the cut cells, one part of a cell per
 // block row: the list is a few blocks, so a thread's chain of loads and
-// atomics is the time (105 and 167 us with whole cells).
+// atomics is the time.  At every size (AS_DIVCUT and AS_RSRC, against whole
+// cells, us: 2.9e3 cells 30 / 81 and 137 / 189, 9.6e3 42 / 88 and 143 / 188,
+// 20e3 66 / 124 and 152 / 199).
 template <int S>
 __global__ void __launch_bounds__(kBlock)
 k_eb_adj_list(const EbAdjEnt *tab, const CutCell *cells, int n, HydroConst hc) {

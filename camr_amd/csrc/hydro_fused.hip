@@ -316,11 +316,12 @@ __device__ __forceinline__ void store_tflux(const CView &F, unsigned v, const do
 // overrides of Hydro_cmpflx.H:239-282 stay in the stored states, because
 // the transverse stages read them.
 //
-// What bounds it (256^3, PPM): waiting for loads, half of a wavefront's
-// time; VALU issue is at 51 %, 18.7 GB of traffic at 3.4 TB/s.  So a wave
-// gets the registers to issue its 47 loads at once (3 waves per SIMD:
-// 5.40 ms per step; 4 waves with loads between the arithmetic 6.00 ms, 5
-// and 6 waves spill: 7.7 and 9.4 ms).  The tile of 16 cells along y or z
+// What bounds it (256^3, PPM): neither rate alone.  18.8 GB of traffic (16.8
+// algorithmic) go at 3.5 TB/s, below a copy's rate, VALU issue is at 48 %, and
+// a wave waits three quarters of its time, half to issue and a quarter for
+// data.  So a wave gets the registers to issue its 47 loads at once (3 waves
+// per SIMD: 5.40 ms per step; 4 waves with loads between the arithmetic 6.00
+// ms, 5 and 6 waves spill: 7.7 and 9.4 ms).  The tile of 16 cells along y or z
 // keeps the 5-point stencil in the CU's own cache: separate launches over
 // rows read 19.5 GB where this reads 6.4 GB, and the first solve no longer
 // reads the 18 state values back.  Traces and first solves as six launches
@@ -2041,6 +2042,9 @@ int fused_umdrv(const UmdrvArgs &A, double dt, double *scratch, hipStream_t st) 
         hipLaunchKernelGGL(k_face1_ppm, grid(T), dim3(kBlock), 0, st, T, hc, dtp);
     else
         hipLaunchKernelGGL(k_face1_plm, grid(T), dim3(kBlock), 0, st, T, has_src, hc, dtp);
+    // the three directions in one launch at every size: hosts cut their grids
+    // at 128^3 and below, where it wins (see kMergeThreads); a 256^3 call (22.3
+    // ms) would gain about what a level of that size does apart, 2 %
     T = three(blocks(ST_T1), blocks(ST_T1 + 1), blocks(ST_T1 + 2));
     hipLaunchKernelGGL(k_trans1_all, grid(T), dim3(kBlock), 0, st, T, hc, dtp);
     // the fluxes go straight into the caller's arrays, or into the canonical

@@ -25,7 +25,8 @@
 // k_fill_fused flags rho < small_dens in raw S_old, k_update_post flags it in
 // S_new, and the level driver then recomputes the step with the unfused
 // sequence from the untouched raw S_old.  Both move at about the rate of a
-// copy (256^3: 4.7 GB in 0.95 ms and 9.4 GB in 1.65 ms).  Constant gravity
+// copy (256^3: 4.6 GB in 0.95 ms and 9.5 GB in 1.65 ms, 1.27 times
+// its algorithmic bytes: about one read of the z fluxes more).  Constant gravity
 // takes the same two passes: 19 pass-by-pass launches of a 97x83x61 step
 // with gravity (0.34 of its 0.97 ms) became 2, 0.76 ms.
 #include "hydro_fused.h"
