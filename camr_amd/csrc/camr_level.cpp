@@ -1588,6 +1588,10 @@ int HydroLevel::construct_hydro_source(double dt, bool add) {
                     return CAMR_ERR_PARAM;
                 }
             }
+            if (!cut_buf_) {
+                set_error("the arrays of the cut-cell boxes could not be allocated");
+                return CAMR_ERR_ALLOC;
+            }
             const int nc = (int)cut_ids_.size();
             int rc = eb_prim_batch(cut_tab_, cut_htab_.data(), nc, hc_, status_, cs, &prof_);
             if (!rc)
@@ -2566,6 +2570,11 @@ int HydroLevel::eb_force_seed(const double w[3]) {
 int HydroLevel::adjoint_backward() {
     const int nsteps = (int)adj_dts_.size();
     if (nsteps == 0 || abar_[0].empty()) { set_error("no adjoint forward run"); return CAMR_ERR_PARAM; }
+    if (ebflags_ && (!eadj_abuf_ || (!cut_ids_.empty() && !cut_buf_))) {
+        // (a later forward run gave them up and failed)
+        set_error("the adjoint's arrays could not be allocated");
+        return CAMR_ERR_ALLOC;
+    }
     const int every = adj_every_;
     const int nck = (nsteps + every - 1) / every;
     int rc = resolve();
@@ -3398,13 +3407,16 @@ namespace {
 // them and void that capture).
 class RelaxedCapture {
   public:
-    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
-    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+    RelaxedCapture() : on_(hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess) {}
+    ~RelaxedCapture() {
+        if (on_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
     RelaxedCapture(const RelaxedCapture &) = delete;
     RelaxedCapture &operator=(const RelaxedCapture &) = delete;
 
   private:
     hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+    bool on_;
 };
 
 // A few words of device memory and their pinned host mirror, for the

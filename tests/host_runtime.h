@@ -2,7 +2,8 @@
 // for tests of the library's host code without a GPU: an executable that
 // includes this and links libcamr_hydro.so has the library call these.
 // Kernels do not run.  fake::cap bounds the "device" memory, fake::fail_at
-// makes the n-th hipMalloc from now on fail (1 = the next).
+// makes the n-th hipMalloc from now on fail (1 = the next), fake::lose_freed the
+// one after every hipFree (as if another program had taken what was freed).
 #pragma once
 
 #define __HIP_PLATFORM_AMD__ 1
@@ -15,6 +16,7 @@
 namespace fake {
 inline size_t cap = size_t(1) << 40, used = 0, peak = 0;
 inline long fail_at = 0, mallocs = 0, launches = 0;
+inline bool lose_freed = false;
 inline std::map<void *, size_t> live;
 inline hipError_t last = hipSuccess;
 } // namespace fake
@@ -38,6 +40,7 @@ hipError_t hipFree(void *p) {
     fake::used -= it->second;
     fake::live.erase(it);
     free(p);
+    if (fake::lose_freed) fake::fail_at = 1;
     return hipSuccess;
 }
 hipError_t hipMemGetInfo(size_t *f, size_t *t) {

@@ -78,9 +78,11 @@ static void mol() {
 // with them; what pair by pair needs is enough, and less than that is refused.
 struct EbRun {
     int made = 0, grad = 0, again = 0;  // return codes of the three
+    int back = 0;                       // of a backward pass on what is left
+    long launched = 0;                  // by it
     size_t peak = 0;
 };
-static EbRun eb(int merge, size_t cap) {
+static EbRun eb(int merge, size_t cap, int lose = 0) {
     const int n = 16;
     const std::vector<int32_t> boxes = {0, 0, 0, 15, 15, 7, 0, 0, 8, 15, 15, 15};
     camr_level_desc d = desc(n, boxes);
@@ -109,7 +111,24 @@ static EbRun eb(int merge, size_t cap) {
         int rc = camr_level_adjoint_forward(L, steps, dts.data(), every);
         return rc ? rc : camr_level_adjoint_backward(L);
     };
-    if (!r.made && !(r.grad = gradient(1, 1))) r.again = gradient(6, 2);
+    if (!r.made && lose) {
+        // what a failed gradient gives up is gone (2: after one that fitted): the
+        // level neither steps nor goes backward on arrays it no longer has
+        if (lose == 2) {
+            CHECK(gradient(1, 1) == CAMR_OK, "first gradient");
+            fake::cap = fake::used;
+        }
+        fake::lose_freed = true;
+        r.grad = camr_level_adjoint_forward(L, 6, dts.data(), 1);
+        fake::lose_freed = false;
+        fake::fail_at = 0;
+        r.again = camr_level_advance(L, 1e-3);
+        fake::launches = 0;
+        r.back = camr_level_adjoint_backward(L);
+        r.launched = fake::launches;
+    } else if (!r.made && !(r.grad = gradient(1, 1))) {
+        r.again = gradient(6, 2);
+    }
     if (!r.made && !r.grad && !r.again) CHECK(fake::last == hipSuccess, "error left");
     if (L) camr_level_destroy(L);
     CHECK(fake::used == 0, "%zu bytes left", fake::used);
@@ -127,6 +146,12 @@ static void eb_levels() {
         const EbRun r = eb(1, cap);
         CHECK(!r.made && !r.grad && !r.again, "%zu of %zu bytes: %d %d %d", cap, full.peak, r.made,
               r.grad, r.again);
+    }
+    for (int lose : {1, 2}) {
+        const EbRun r = eb(1, lose == 1 ? lean.peak + (full.peak - lean.peak) / 4 : fake::cap, lose);
+        CHECK(!r.made && r.grad && r.again == CAMR_ERR_ALLOC, "%d: %d %d %d", lose, r.made, r.grad,
+              r.again);
+        CHECK(r.back && r.launched == 0, "%d: %d after %ld launches", lose, r.back, r.launched);
     }
     for (int merge = 0; merge < 2; ++merge)
         for (int s = 1; s < 40; ++s) {
