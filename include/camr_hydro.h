@@ -240,10 +240,11 @@ int camr_level_set_stream(camr_level *L, void *stream);
 int camr_level_upload_box(camr_level *L, int32_t b, const double *host);
 int camr_level_download_box(camr_level *L, int32_t b, double *host);
 /* Device view of the new-time state of box b (valid cells, NVAR comps).
- * Waits for a step of the fused engine that is still running: where a density
- * floor acts, the level redoes that step, and a view taken earlier holds the
- * final state only after this call, camr_level_sync or one that reads the
- * state.  Returns the step's error if it had one. */
+ * Where a density floor acts in a step of the fused engine, the level redoes
+ * that step when it next waits for it: a view holds the final state after
+ * camr_level_sync, _new_dt or any call that reads the state, before that the
+ * state without the floors.  On a level with gravity this call waits itself,
+ * and returns the step's error if it had one. */
 int camr_level_state_array(camr_level *L, int32_t b, camr_array4 *out);
 /* CAMR::initData tail: enforce_consistent_e + computeTemp (CAMR.cpp:423-425). */
 int camr_level_init_post(camr_level *L);
